@@ -434,12 +434,37 @@ __device__ __forceinline__ float row_multiplier(float absmax) {
   return absmax > 0.0f ? 127.0f / absmax : 1.0f;
 }
 
+// 1 / x for a positive x in [2^-125, 2^126): the hardware's estimate and one
+// Newton step.  Equal to the IEEE quotient on every float of that range (all
+// 2^31 of them compared on the device), three instructions instead of the
+// division's ten.
+__device__ __forceinline__ float recip_exact(float x) {
+  const float r = __builtin_amdgcn_rcpf(x);
+  return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);
+}
+// Whether v is positive with an exponent in [-62, 62): two such factors have
+// a product within recip_exact's range.
+__device__ __forceinline__ bool recip_factor(float v) {
+  return __float_as_uint(v) - (65u << 23) < (124u << 23);
+}
+
 // y = acc * (1 / (a * w)) + b: one multiply, one divide, one multiply, one add
 // (q8_gemm.rs:438-446).
 __device__ __forceinline__ float dequant_scale(float a, float w) { return 1.0f / (a * w); }
 __device__ __forceinline__ float dequant_apply(int32_t acc, float inv, float b) { return (float)acc * inv + b; }
 __device__ __forceinline__ float dequant(int32_t acc, float a, float w, float b) {
   return dequant_apply(acc, dequant_scale(a, w), b);
+}
+
+// v where keep holds, else zero, with v's load issued either way (its address
+// must be valid).  The mask goes through an empty asm so that the compiler
+// cannot turn the choice back into a select, which it lowers to a branch
+// around the load; a load behind a branch is waited for inside it, which
+// serializes the loads issued before and after it.
+__device__ __forceinline__ v4i keep_or_zero(v4i v, bool keep) {
+  int m = keep ? -1 : 0;
+  asm("" : "+v"(m));
+  return v & v4i{m, m, m, m};
 }
 
 // Weights in MFMA fragment order: for the 16-column tile t and the 64-wide

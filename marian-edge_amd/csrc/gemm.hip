@@ -21,17 +21,6 @@ constexpr int kSkinnyMaxK = 2048;  // 8 waves x 4 k-steps x 64
 
 
 __device__ __forceinline__ v4i zero4() { return v4i{0, 0, 0, 0}; }
-// v where keep holds, else zero, with v's load issued either way (its address
-// must be valid).  The mask goes through an empty asm so that the compiler
-// cannot turn the choice back into a select, which it lowers to a branch
-// around the load; a load behind a branch is waited for inside it, which
-// serializes the loads issued before and after it.
-__device__ __forceinline__ v4i keep_or_zero(v4i v, bool keep) {
-  int m = keep ? -1 : 0;
-  asm("" : "+v"(m));
-  return v & v4i{m, m, m, m};
-}
-
 // ---------------------------------------------------------------------------
 // Skinny GEMM (decode and small M).  One workgroup owns CT*16 output columns
 // for every row; its NW waves split K (wave w takes k-steps w, w+NW, ...),
@@ -562,190 +551,6 @@ __global__ __launch_bounds__(64 * kVocabWaves<LNP>) void k_vocab_argmax(GemmArgs
 }
 
 // ---------------------------------------------------------------------------
-// Tile GEMM: 64x64 output tile per workgroup, 4 waves in a 2x2 grid each
-// owning 32x32 (2x2 MFMA tiles).  K is staged through LDS in chunks of up to
-// 512: the whole chunk of both operands is requested at once (64 KB per
-// workgroup in flight), and the next chunk's loads are in flight while the
-// MFMAs consume the current one, so a K of 512 costs one memory round trip
-// instead of one per 64-wide k-step.  The epilogue dequantizes into LDS and
-// stores whole 256-byte row segments.
-//
-// Tile order: the grid is one-dimensional and workgroups reach the 8 XCDs
-// round-robin, so the linear id is remapped to give each XCD a contiguous
-// range of tiles, with the column tile varying fastest.  The workgroups in
-// flight on one XCD then share their activation rows (in its L2) and write
-// adjacent 256-byte pieces of the same output rows: the output is most of
-// the traffic, and the row tile varying fastest (writes spread over many
-// rows at once) measured 15% slower on 4096 x 32000.  Grids more than
-// kTileWideN column tiles wide take the column tiles in groups of
-// kTileGroup row tiles (row tile fastest within a group), so a weight tile
-// is fetched into an XCD's L2 once for eight row tiles instead of once per
-// row tile (4096 x 32000: 360 -> 344 us with both outputs, 272 -> 253 us
-// with the fp32 one; the narrow encoder shapes keep their weights in L2
-// either way and were within noise).
-// The output rows are written with non-temporal stores (they are not read
-// again by this kernel): 3-14% faster from M = 1400 to 7400 on the encoder
-// and op-level shapes.
-// ---------------------------------------------------------------------------
-constexpr int kTm = 64;         // tile edge (rows and columns)
-constexpr int64_t kTileBigGrid = 256;  // tiles above which K chunks are 256 wide
-constexpr int kTout = kTm + 4;  // padded LDS row of the epilogue (words)
-constexpr int kTileWideN = 64;  // column tiles above which tiles go in row groups
-constexpr int kTileGroup = 8;   // row tiles per group
-
-template <int KC>  // K chunk staged in LDS: 512 (one round trip for K = 512) or 256
-__global__ __launch_bounds__(256) void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
-  constexpr int LDS_ROW = KC + 16;                // padded LDS row (bytes)
-  constexpr int ROW_CH = KC / 16;                 // 16-byte pieces per row
-  constexpr int CH = kTm * ROW_CH / 256;          // 16-byte loads per thread per operand
-  static_assert(kTm * LDS_ROW >= kTm * kTout * 4, "the epilogue reuses the operand tiles");
-  __shared__ __attribute__((aligned(16))) int8_t sA[kTm * LDS_ROW];
-  __shared__ __attribute__((aligned(16))) int8_t sB[kTm * LDS_ROW];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int wm = wave >> 1, wn = wave & 1;
-  int tile = blockIdx.x;
-  const int full = tiles & ~7;
-  if (tile < full) tile = (tile & 7) * (full >> 3) + (tile >> 3);
-  const int M = g.M, N = g.N, K = g.K;
-  int m0 = tile / tiles_n * kTm, n0 = tile % tiles_n * kTm;
-  if (tiles_n > kTileWideN) {  // a permutation of the tiles: groups of up to kTileGroup row tiles
-    const int tiles_m = (M + kTm - 1) / kTm;
-    const int grp = tile / (kTileGroup * tiles_n), first_m = grp * kTileGroup;
-    const int gm = min(kTileGroup, tiles_m - first_m), in_g = tile - grp * kTileGroup * tiles_n;
-    m0 = (first_m + in_g % gm) * kTm;
-    n0 = in_g / gm * kTm;
-  }
-
-  // Every load is issued (from an in-bounds address); pieces past M, N or
-  // the chunk's K are zeroed when they are stored to LDS.
-  v4i ra[CH], rb[CH];
-  bool ka[CH], kb[CH];
-  auto gload = [&](int k0, int kc) {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c = tid + i * 256, row = c / ROW_CH, col = c % ROW_CH * 16;
-      const int m = m0 + row, n = n0 + row;
-      const int cl = min(col, kc - 16);
-      ra[i] = *(const v4i*)(g.A + (int64_t)min(m, M - 1) * g.lda + k0 + cl);
-      rb[i] = *(const v4i*)(g.W + (int64_t)min(n, N - 1) * K + k0 + cl);
-      ka[i] = col < kc && m < M;
-      kb[i] = col < kc && n < N;
-    }
-  };
-  auto lstore = [&]() {
-#pragma unroll
-    for (int i = 0; i < CH; ++i) {
-      const int c = tid + i * 256, row = c / ROW_CH, col = c % ROW_CH * 16;
-      *(v4i*)(sA + row * LDS_ROW + col) = keep_or_zero(ra[i], ka[i]);
-      *(v4i*)(sB + row * LDS_ROW + col) = keep_or_zero(rb[i], kb[i]);
-    }
-  };
-
-  v4i acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = zero4();
-
-  const int kq = (lane >> 4) * 16;
-  const int8_t* pa = sA + (wm * 32 + (lane & 15)) * LDS_ROW + kq;
-  const int8_t* pb = sB + (wn * 32 + (lane & 15)) * LDS_ROW + kq;
-  gload(0, min(KC, K));
-  lstore();
-  __syncthreads();
-  for (int k0 = 0; k0 < K; k0 += KC) {
-    const int ksteps = min(KC, K - k0) >> 6;
-    const bool more = k0 + KC < K;
-    if (more) gload(k0 + KC, min(KC, K - k0 - KC));
-#pragma unroll
-    for (int ks = 0; ks < KC / 64; ++ks) {
-      if (ks < ksteps) {
-        const v4i a0 = *(const v4i*)(pa + ks * 64);
-        const v4i a1 = *(const v4i*)(pa + 16 * LDS_ROW + ks * 64);
-        const v4i b0 = *(const v4i*)(pb + ks * 64);
-        const v4i b1 = *(const v4i*)(pb + 16 * LDS_ROW + ks * 64);
-        acc[0][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b0, acc[0][0], 0, 0, 0);
-        acc[0][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, b1, acc[0][1], 0, 0, 0);
-        acc[1][0] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b0, acc[1][0], 0, 0, 0);
-        acc[1][1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1, b1, acc[1][1], 0, 0, 0);
-      }
-    }
-    if (more) {
-      __syncthreads();
-      lstore();
-      __syncthreads();
-    }
-  }
-
-  // Epilogue: element (m, n) of the MFMA tile (i, j) is register r of lane
-  // (m % 16 / 4) * 16 + n % 16 with r = m % 4.
-  float arow[2][4];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = m0 + wm * 32 + i * 16 + (lane >> 4) * 4 + r;
-      arow[i][r] = m < M ? g.a[m] : 1.0f;
-    }
-  float* sO = (float*)sA;      // [kTm][kTout] dequantized
-  int32_t* sI = (int32_t*)sB;  // [kTm][kTout] accumulators
-  __syncthreads();             // the MFMAs' last LDS reads are done
-#pragma unroll
-  for (int j = 0; j < 2; ++j) {
-    const int nl = wn * 32 + j * 16 + (lane & 15), n = n0 + nl;
-    const float wmul = n < N ? g.wmult[n] : 1.0f, bias = n < N ? g.bias[n] : 0.0f;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int ml = wm * 32 + i * 16 + (lane >> 4) * 4 + r;
-        const int32_t iv = acc[i][j][r];
-        float y = dequant(iv, arow[i][r], wmul, bias);
-        if (e.relu) y = y > 0.0f ? y : 0.0f;
-        sO[ml * kTout + nl] = y;
-        sI[ml * kTout + nl] = iv;
-      }
-  }
-  __syncthreads();
-  const bool vec_o = e.out && (e.ldo & 3) == 0 && ((uintptr_t)e.out & 15) == 0;
-  const bool vec_i = e.out_i32 && (e.ldi & 3) == 0 && ((uintptr_t)e.out_i32 & 15) == 0;
-#pragma unroll
-  for (int q = 0; q < kTm * kTm / 4 / 256; ++q) {
-    const int idx = tid + q * 256, row = idx >> 4, c4 = (idx & 15) * 4;
-    const int m = m0 + row, n = n0 + c4;
-    if (m >= M || n >= N) continue;
-    const float* so = sO + row * kTout + c4;
-    const int32_t* si = sI + row * kTout + c4;
-    if (e.out) {
-      float* o = e.out + (int64_t)m * e.ldo + n;
-      if (vec_o && n + 4 <= N) {
-        __builtin_nontemporal_store(*(const f4v*)so, (f4v*)o);
-      } else {
-        for (int t = 0; t < 4 && n + t < N; ++t) o[t] = so[t];
-      }
-    }
-    if (e.out_i32) {
-      int32_t* o = e.out_i32 + (int64_t)m * e.ldi + n;
-      if (vec_i && n + 4 <= N) {
-        __builtin_nontemporal_store(*(const v4i*)si, (v4i*)o);
-      } else {
-        for (int t = 0; t < 4 && n + t < N; ++t) o[t] = si[t];
-      }
-    }
-    if (e.out_q) {
-      int8_t* o = e.out_q + (int64_t)m * e.ldq + n;
-      bool bad = false;
-      for (int t = 0; t < 4 && n + t < N; ++t) {
-        o[t] = (int8_t)quantize_one(so[t], e.qmult);
-        bad |= !isfinite(so[t]);
-      }
-      if (n == 0) e.out_qa[m] = e.qmult;
-      if (bad && g.err) *g.err = 1;  // quantizing rejects non-finite input
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // Output scoring over a candidate list (the lexical shortlist's ids, sorted
 // ascending): select_token (q8_engine.rs:749-790) for row m scores only
 // cand[off[m] .. off[m+1]).  One workgroup per (row, 128 candidates): each of
@@ -1004,26 +809,6 @@ hipError_t launch_vocab_argmax(const GemmArgs& g, const Epilogue& e, hipStream_t
     hipExtLaunchKernelGGL(kern, grid, block, 0, s, ev_start, ev_stop, 0, g, e);
   else
     hipLaunchKernelGGL(kern, grid, block, 0, s, g, e);
-  return hipGetLastError();
-}
-
-hipError_t launch_gemm_tile(const GemmArgs& g, const Epilogue& e, hipStream_t s) {
-  if (g.K <= 0 || g.K % 64 || g.N <= 0 || g.M_dev || g.lda % 16) return hipErrorInvalidValue;
-  if (e.out_q && (!e.out_qa || e.ldq < g.N || !(e.qmult > 0.0f) || !(e.qmult < __builtin_huge_valf())))
-    return hipErrorInvalidValue;
-  if (g.M <= 0) return hipSuccess;
-  const int64_t tiles = (int64_t)((g.M + kTm - 1) / kTm) * ((g.N + kTm - 1) / kTm);
-  if (tiles > (int64_t)INT32_MAX) return hipErrorInvalidValue;
-  const int tiles_n = (g.N + kTm - 1) / kTm;
-  // Launches of more than one round of 512-wide-chunk workgroups (two per
-  // CU) take the 256-wide chunks (34 KB of LDS, four workgroups per CU, more
-  // loads in flight per CU: 385 vs 469 us on 4096 x 32000; the encoder's QKV
-  // and FFN1 in one round instead of two); smaller ones the 512-wide chunks
-  // (one round trip for K = 512).
-  if (tiles > kTileBigGrid)
-    hipLaunchKernelGGL(k_gemm_tile<256>, dim3((unsigned)tiles), dim3(256), 0, s, g, e, tiles_n, (int)tiles);
-  else
-    hipLaunchKernelGGL(k_gemm_tile<512>, dim3((unsigned)tiles), dim3(256), 0, s, g, e, tiles_n, (int)tiles);
   return hipGetLastError();
 }
 

@@ -1,0 +1,303 @@
+// tile.hip — LDS-tiled int8 MFMA GEMM for many rows (v_mfma_i32_32x32x32_i8).
+//
+// Operands and epilogue are those of gemm.hip: activations A[M, K] and weights
+// W[N, K], both K-contiguous, exact i32 accumulators, y = acc * (1/(a_m w_n)) +
+// b_n with optional ReLU, i32 copy and statically quantized copy.
+#include "device_common.h"
+#include "kernels.h"
+#include <algorithm>
+
+namespace mh {
+namespace {
+
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+// ---------------------------------------------------------------------------
+// One workgroup of WM x WN waves per BM x BN output tile, each wave a grid of
+// 32x32 MFMA blocks.  K moves in 128-byte chunks: registers hold the next PF
+// chunks (requested that far ahead, across tile boundaries too: a workgroup
+// walks several tiles, so the next tile's first chunks arrive while this
+// tile's results are dequantized and stored), LDS two, one barrier per chunk.
+//
+// LDS rows are 128 bytes, the 16-byte piece p of row r at slot p ^ (r % 8), so
+// that both the stores (eight lanes per row) and the MFMA operand reads (32
+// rows, one piece each) touch every bank equally.
+//
+// Lane l of an output block holds column l % 32 and rows 8(r/4) + 4(l/32) +
+// r%4 (register r): a store instruction writes two whole 128-byte lines
+// straight from the accumulators, with no pass through LDS.
+//
+// Tile order: workgroups reach the 8 XCDs round-robin; each XCD takes a
+// contiguous range of tiles.  Wide outputs go in groups of kTileGroup row
+// tiles (row tile fastest), so a weight tile reaches an XCD's L2 once per
+// group; narrow ones column tile fastest, so activations are shared.
+//
+// What bounds it (4096 x 32000, K = 512, 256x128 tiles, one workgroup per CU):
+// 134 us against 236 us for the 64x64 tiles it replaces, which divided in the
+// epilogue and staged every result through LDS.  The epilogue with its stores
+// alone takes 105 us (5.0 TB/s of output), the K loop alone under 90 us; the
+// rest is what the two do not overlap.  At 1459 x 512 (K = 512) a tile's
+// memory round trip and the dispatch are 5.1 us (6.3 before).
+// ---------------------------------------------------------------------------
+constexpr int kTileKC = 128;     // bytes of K per chunk
+constexpr int kTileGroup = 8;    // row tiles per group
+constexpr int kTileWideN = 32;   // column tiles above which tiles go in groups
+
+// Output rows [0, rows) of a tile as a raw buffer (empty without an output):
+// stores at or past its end are dropped.
+constexpr int kRawBufferWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
+constexpr int kNt = 2;                       // non-temporal: the outputs are not read again here
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const void* p, int64_t elem0, int64_t ld, int rows,
+                                                            int size) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)((const char*)p + (p ? elem0 * size : 0)), (short)0,
+                                           p ? (int)(rows * ld * size) : 0, kRawBufferWord3);
+}
+
+template <int BM, int BN, int WM, int WN, int PF, bool RELU, bool EXTRA, bool WIDE>
+__global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(BM > 128 ? 2 : WM * WN / 2)))
+void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
+  constexpr int NT = WM * WN * 64;
+  constexpr int MB = BM / WM / 32, NB = BN / WN / 32;  // 32x32 blocks per wave
+  constexpr int AP = BM * 8 / NT, BP = BN * 8 / NT;    // 16-byte pieces per thread and chunk
+  static_assert(AP * NT == BM * 8 && BP * NT == BN * 8 && PF % 2 == 0, "whole pieces, even ring");
+  static_assert(NT >= BM, "a thread per row multiplier");
+  __shared__ __attribute__((aligned(16))) int8_t sA[2][BM * kTileKC];
+  __shared__ __attribute__((aligned(16))) int8_t sB[2][BN * kTileKC];
+  __shared__ float sAm[2][BM];
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WN * (BM / WM), wc = wave % WN * (BN / WN);  // the wave's corner
+  const int M = g.M, N = g.N, K = g.K;
+
+  // This workgroup's tiles: lo + slot, + per_xcd, ... below hi.
+  const int xcd = blockIdx.x & 7, per_xcd = (gridDim.x + 7) >> 3;
+  const int hi = (int)((int64_t)(xcd + 1) * tiles >> 3);
+  const int first = (int)((int64_t)xcd * tiles >> 3) + (blockIdx.x >> 3);
+  if (first >= hi) return;  // the whole workgroup
+  auto corner = [&](int tile, int& m0, int& n0) {
+    if (tiles_n > kTileWideN) {
+      const int tiles_m = (M + BM - 1) / BM;
+      const int grp = tile / (kTileGroup * tiles_n), first_m = grp * kTileGroup;
+      const int gm = min(kTileGroup, tiles_m - first_m), in_g = tile - grp * kTileGroup * tiles_n;
+      m0 = (first_m + in_g % gm) * BM;
+      n0 = in_g / gm * BN;
+    } else {
+      m0 = tile / tiles_n * BM;
+      n0 = tile % tiles_n * BN;
+    }
+  };
+
+  // The loader runs PF chunks ahead and is branch-free: past a tile's last
+  // chunk it goes on with the next tile (the last tile again at the end), rows
+  // past M or N reload the last one (their results are not stored) and pieces
+  // past K reload the row's last piece; A's are zeroed at the LDS store.  A
+  // tile counts a multiple of PF chunks, so a chunk's registers and LDS buffer
+  // are fixed at compile time.
+  const int nslot = (K + kTileKC * PF - 1) / (kTileKC * PF) * PF;
+  v4i ra[PF][AP], rb[PF][BP];
+  const int8_t *pa[AP], *pb[BP];
+  const int kp = (tid & 7) * 16;  // this thread's piece of each chunk
+  auto point = [&](int m0, int n0) {
+#pragma unroll
+    for (int i = 0; i < AP; ++i) pa[i] = g.A + (int64_t)min(m0 + ((tid + i * NT) >> 3), M - 1) * g.lda;
+#pragma unroll
+    for (int i = 0; i < BP; ++i) pb[i] = g.W + (int64_t)min(n0 + ((tid + i * NT) >> 3), N - 1) * K;
+  };
+  auto gload = [&](int c, v4i (&xa)[AP], v4i (&xb)[BP]) {
+    const int col = min(c * kTileKC + kp, K - 16);
+#pragma unroll
+    for (int i = 0; i < AP; ++i) xa[i] = *(const v4i*)(pa[i] + col);
+#pragma unroll
+    for (int i = 0; i < BP; ++i) xb[i] = *(const v4i*)(pb[i] + col);
+  };
+  int m0, n0;
+  corner(first, m0, n0);
+  point(m0, n0);
+#pragma unroll
+  for (int u = 0; u < PF; ++u) gload(u, ra[u], rb[u]);
+
+  int tpar = 0;
+  for (int tile = first; tile < hi; tile += per_xcd, tpar ^= 1) {
+    int m1 = m0, n1 = n0;  // the next tile's corner
+    v16i acc[MB][NB];
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int k = 0; k < NB; ++k)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][k][r] = 0;
+    // The tile's row multipliers (into LDS with its chunks) and this lane's
+    // column operands: both arrive under the products.
+    const float am = g.a[min(m0 + min(tid, BM - 1), M - 1)];
+    float wm[NB], bi[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      const int n = min(n0 + wc + k * 32 + (lane & 31), N - 1);
+      wm[k] = g.wmult[n];
+      bi[k] = g.bias[n];
+    }
+    for (int c0 = 0; c0 < nslot; c0 += PF) {
+      int cl = c0 + PF;  // the chunks to request
+      if (cl == nslot) {
+        if (tile + per_xcd < hi) corner(tile + per_xcd, m1, n1);
+        point(m1, n1);
+        cl = 0;
+        if (tid < BM) sAm[tpar][tid] = am;
+      }
+#pragma unroll
+      for (int u = 0; u < PF; ++u) {
+        const bool in_k = (c0 + u) * kTileKC + kp < K;
+#pragma unroll
+        for (int i = 0; i < AP; ++i) {
+          const int c = tid + i * NT, row = c >> 3;
+          *(v4i*)(sA[u & 1] + row * kTileKC + (((c & 7) ^ (row & 7)) << 4)) = keep_or_zero(ra[u][i], in_k);
+        }
+#pragma unroll
+        for (int i = 0; i < BP; ++i) {
+          const int c = tid + i * NT, row = c >> 3;
+          *(v4i*)(sB[u & 1] + row * kTileKC + (((c & 7) ^ (row & 7)) << 4)) = rb[u][i];
+        }
+        gload(cl + u, ra[u], rb[u]);
+        wg_lds_barrier();
+        const int8_t* la = sA[u & 1] + (wr + (lane & 31)) * kTileKC;
+        const int8_t* lb = sB[u & 1] + (wc + (lane & 31)) * kTileKC;
+#pragma unroll
+        for (int ks = 0; ks < kTileKC / 32; ++ks) {
+          const int at = ((2 * ks + half) ^ (lane & 7)) << 4;
+          v4i fa[MB], fb[NB];
+#pragma unroll
+          for (int i = 0; i < MB; ++i) fa[i] = *(const v4i*)(la + i * 32 * kTileKC + at);
+#pragma unroll
+          for (int k = 0; k < NB; ++k) fb[k] = *(const v4i*)(lb + k * 32 * kTileKC + at);
+#pragma unroll
+          for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int k = 0; k < NB; ++k)
+              acc[i][k] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[k], acc[i][k], 0, 0, 0);
+        }
+      }
+    }
+    // ---- epilogue ----
+    bool ok = true;
+#pragma unroll
+    for (int i = 0; i < BM; i += 64) ok &= recip_factor(sAm[tpar][i + lane]);
+#pragma unroll
+    for (int k = 0; k < NB; ++k) ok &= recip_factor(wm[k]);
+    ok = __all(ok);
+    const float* sm = sAm[tpar] + wr + 4 * half;
+    const int rows = min(BM, M - m0);
+    const uint32_t row0 = (uint32_t)(wr + 4 * half);
+    // Buffer stores whose range ends with the tile's last row drop the rows
+    // past M; a lane past N starts past the range.
+    const __amdgpu_buffer_rsrc_t ro = tile_rows(e.out, (int64_t)m0 * e.ldo, e.ldo, rows, 4);
+    const __amdgpu_buffer_rsrc_t ri = tile_rows(EXTRA ? e.out_i32 : nullptr, (int64_t)m0 * e.ldi, e.ldi, rows, 4);
+    const __amdgpu_buffer_rsrc_t rq = tile_rows(EXTRA ? e.out_q : nullptr, (int64_t)m0 * e.ldq, e.ldq, rows, 1);
+    bool bad = false;
+    int ncol[NB];
+    uint32_t off[NB];
+#pragma unroll
+    for (int k = 0; k < NB; ++k) {
+      ncol[k] = n0 + wc + k * 32 + (lane & 31);
+      off[k] = ncol[k] < N ? (row0 * (uint32_t)e.ldo + (uint32_t)ncol[k]) * 4u : 0x80000000u;
+    }
+#pragma unroll
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 a4 = *(const float4*)(sm + i * 32 + 8 * q);
+        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+        float inv[4][NB];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int k = 0; k < NB; ++k) inv[r][k] = recip_exact(av[r] * wm[k]);
+        if (!ok) {  // a multiplier outside recip_exact's range: the IEEE quotient
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int k = 0; k < NB; ++k) inv[r][k] = dequant_scale(av[r], wm[k]);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t ml = row0 + (uint32_t)(i * 32 + 8 * q + r);  // row of the tile
+#pragma unroll
+          for (int k = 0; k < NB; ++k) {
+            const int32_t iv = acc[i][k][4 * q + r];
+            float y = dequant_apply(iv, inv[r][k], bi[k]);
+            if (RELU) y = y > 0.0f ? y : 0.0f;
+            if constexpr (!EXTRA) {
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ro, off[k], 0, kNt);
+              off[k] += (r == 3 ? 5u : 1u) * (uint32_t)e.ldo * 4u;  // rows 0-3, 8-11, 16-19, 24-27 of each block
+            } else if (WIDE) {  // row strides past the buffer offsets
+              const int64_t m = m0 + (int64_t)ml;
+              if (m < M && ncol[k] < N) {
+                if (e.out) e.out[m * e.ldo + ncol[k]] = y;
+                if (e.out_i32) e.out_i32[m * e.ldi + ncol[k]] = iv;
+                if (e.out_q) e.out_q[m * e.ldq + ncol[k]] = (int8_t)quantize_one(y, e.qmult);
+                bad |= !isfinite(y);
+              }
+            } else {
+              const bool in = ncol[k] < N;
+              const uint32_t n = (uint32_t)ncol[k];
+              if (e.out)
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ro,
+                                                      in ? (ml * (uint32_t)e.ldo + n) * 4u : 0x80000000u, 0, kNt);
+              if (e.out_i32)
+                __builtin_amdgcn_raw_buffer_store_b32((uint32_t)iv, ri,
+                                                      in ? (ml * (uint32_t)e.ldi + n) * 4u : 0x80000000u, 0, kNt);
+              if (e.out_q)
+                __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(int8_t)quantize_one(y, e.qmult), rq,
+                                                     in ? ml * (uint32_t)e.ldq + n : 0x80000000u, 0, 0);
+              bad |= in && (int)ml < rows && !isfinite(y);
+            }
+          }
+        }
+      }
+    if constexpr (EXTRA) {
+      if (e.out_q) {
+        if (n0 == 0 && tid < rows) e.out_qa[m0 + tid] = e.qmult;
+        if (__any(bad) && lane == 0 && g.err) *g.err = 1;  // quantizing rejects non-finite input
+      }
+    }
+    m0 = m1;
+    n0 = n1;
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int PF, bool WIDE = false>
+hipError_t launch_tile(const GemmArgs& g, const Epilogue& e, int max_wgs, hipStream_t s) {
+  const int64_t tiles_m = (g.M + BM - 1) / BM, tiles_n = (g.N + BN - 1) / BN, tiles = tiles_m * tiles_n;
+  if (tiles > (int64_t)INT32_MAX / 2) return hipErrorInvalidValue;
+  const int grid = (int)std::min<int64_t>((tiles + 7) / 8 * 8, max_wgs);
+  const bool extra = WIDE || e.out_i32 || e.out_q || !e.out;
+  auto kern = e.relu ? (extra ? k_gemm_tile<BM, BN, WM, WN, PF, true, true, WIDE> : k_gemm_tile<BM, BN, WM, WN, PF, true, WIDE, WIDE>)
+                     : (extra ? k_gemm_tile<BM, BN, WM, WN, PF, false, true, WIDE> : k_gemm_tile<BM, BN, WM, WN, PF, false, WIDE, WIDE>);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(WM * WN * 64), 0, s, g, e, (int)tiles_n, (int)tiles);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_gemm_tile(const GemmArgs& g, const Epilogue& e, hipStream_t s) {
+  if (g.K <= 0 || g.K % 64 || g.N <= 0 || g.M_dev || g.lda % 16) return hipErrorInvalidValue;
+  if (e.out_q && (!e.out_qa || e.ldq < g.N || !(e.qmult > 0.0f) || !(e.qmult < __builtin_huge_valf())))
+    return hipErrorInvalidValue;
+  if (g.M <= 0) return hipSuccess;
+  // Buffer offsets of a tile's rows stay below 2^30 (a lane past N starts at
+  // 2^31, above every range); longer rows take 64-bit addresses.
+  if (std::max(std::max(e.out ? e.ldo : 0, e.out_i32 ? e.ldi : 0), e.out_q ? e.ldq : 0) >= (1 << 20))
+    return launch_tile<64, 64, 2, 2, 2, true>(g, e, 1024, s);
+  // By the tiles a shape gives 256 CUs (kernel times in us, this kernel's
+  // sizes in the order 64x64 / 128x128 / 256x128):
+  //   below 224 128x128 tiles, one tile's latency decides and small tiles win:
+  //     1459 x 512 (K 512) 5.1 / 6.9 / 9.3, 4096 x 512 (K 2048) 12.0 / 14.1 / 19.8;
+  //   above, larger tiles read less per output: 7405 x 512 (K 2048) 17.8 / 14.4 /
+  //     19.3, 1000 x 32000 44.9 / 34.0 / 36.9;
+  //   from 2048 256x128 tiles (eight a CU) the largest: 4096 x 32000 175 / 157 / 134.
+  const auto tiles = [&](int64_t bm, int64_t bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+  if (tiles(256, 128) >= 2048) return launch_tile<256, 128, 4, 2, 2>(g, e, 256, s);
+  if (tiles(128, 128) >= 224) return launch_tile<128, 128, 2, 4, 2>(g, e, 1 << 30, s);
+  return launch_tile<64, 64, 2, 2, 2>(g, e, 1024, s);
+}
+
+}  // namespace mh

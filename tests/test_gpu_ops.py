@@ -67,6 +67,52 @@ def test_q8_linear_long_k_row_groups(pkg, orc, dev, M, K, N):
     assert np.array_equal(df.host().view(np.uint32), y_ref.view(np.uint32))
 
 
+def _dequant_ref(acc, a, mult, bias, relu=False):
+    inv = np.float32(1) / (a[:, None] * mult[None, :])
+    y = acc.astype(np.float32) * inv + bias[None, :]
+    return np.where(y > 0, y, np.float32(0)) if relu else y
+
+
+@pytest.mark.parametrize("M,K,N", [
+    (65, 64, 31), (64 * 3 + 1, 192, 129), (127, 2112, 64),  # 64x64 tiles, odd chunk counts, ragged edges
+    (1793, 320, 2047), (1920, 128, 1900),                   # 128x128 tiles: from 224 of them
+    (2305, 64, 29057),                                      # 256x128 tiles: from 2048, the last row tile of one row
+    (65, 64, (1 << 20) + 8),                                # output rows past the buffer stores' offsets
+])
+def test_q8_linear_tile_sizes(dev, M, K, N):
+    """Every tile size of the many-row GEMM at its edges, bit-identical to the
+    integer product (exact in float64) dequantized in fp32; every seventh column and
+    one row with a multiplier outside the fast reciprocal's range."""
+    print(f"q8_linear tiles M={M} K={K} N={N}", flush=True)
+    rng = np.random.default_rng(M + N)
+    q = rng.integers(-127, 128, size=(M, K)).astype(np.int8)
+    w = rng.integers(-127, 128, size=(N, K)).astype(np.int8)
+    a = rng.uniform(20, 60, size=M).astype(np.float32)
+    mult = rng.uniform(50, 100, size=N).astype(np.float32)
+    if N < 4096:
+        mult[3::7] = np.float32(1e-25)
+        a[M // 2] = np.float32(3e25)
+    bias = rng.standard_normal(N).astype(np.float32)
+    # |acc| <= 127^2 K < 2^24 up to K = 1040: exact in fp32 there
+    dt = np.float32 if K <= 1040 else np.float64
+    acc = (q.astype(dt) @ w.astype(dt).T).astype(np.int32)
+    D = dev.DeviceArray
+    dq, dw, da, dm, db = (D.from_host(x) for x in (q, w, a, mult, bias))
+    di, df = D.zeros((M, N), np.int32) if N < 4096 else None, D.zeros((M, N), np.float32)
+    for relu in (False, True) if N < 4096 else (False,):
+        want = _dequant_ref(acc, a, mult, bias, relu)
+        df.fill_bytes(0xFF)
+        dev.q8_linear(None, dw, dm, db, None, df, relu=relu, xq=dq, xa=da)
+        dev.synchronize()
+        assert np.array_equal(df.host().view(np.uint32), want.view(np.uint32)), f"fp32 relu={relu}"
+        if di is not None:
+            df.fill_bytes(0xFF)
+            dev.q8_linear(None, dw, dm, db, di, df, relu=relu, xq=dq, xa=da)
+            dev.synchronize()
+            assert np.array_equal(di.host(), acc)
+            assert np.array_equal(df.host().view(np.uint32), want.view(np.uint32)), f"both relu={relu}"
+
+
 def test_q8_linear_on_two_streams_at_once(pkg, orc, dev):
     """The op-level entry points keep their intermediate buffers (here the
     quantized activations of an fp32 input) per (device, stream): two streams
