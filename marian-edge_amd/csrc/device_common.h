@@ -429,6 +429,24 @@ __device__ __forceinline__ int quantize_one(float x, float a) {
   return (int)v;
 }
 
+// Four values quantized with multiplier a, packed in order (the same integers
+// as quantize_one: clamping first leaves +-127 and rounding to even as they
+// are, and adding 1.5 * 2^23 rounds a value of that size to the integer its
+// low byte then holds), at 3.75 instructions a value.
+__device__ __forceinline__ uint32_t quantize_pack4(float x, float y, float z, float w, float a) {
+  const float b = 12582912.0f;
+  const uint32_t qx = __float_as_uint(__builtin_amdgcn_fmed3f(x * a, -127.0f, 127.0f) + b);
+  const uint32_t qy = __float_as_uint(__builtin_amdgcn_fmed3f(y * a, -127.0f, 127.0f) + b);
+  const uint32_t qz = __float_as_uint(__builtin_amdgcn_fmed3f(z * a, -127.0f, 127.0f) + b);
+  const uint32_t qw = __float_as_uint(__builtin_amdgcn_fmed3f(w * a, -127.0f, 127.0f) + b);
+  const uint32_t xy = __builtin_amdgcn_perm(qy, qx, 0x0c0c0400);  // bytes x, y
+  const uint32_t zw = __builtin_amdgcn_perm(qw, qz, 0x04000c0c);  // bytes z, w in the upper half
+  return xy | zw;
+}
+__device__ __forceinline__ uint32_t quantize_pack4(float4 v, float a) {
+  return quantize_pack4(v.x, v.y, v.z, v.w, a);
+}
+
 // Per-row activation multiplier: 127 / max|x| (1 for an all-zero row).
 __device__ __forceinline__ float row_multiplier(float absmax) {
   return absmax > 0.0f ? 127.0f / absmax : 1.0f;

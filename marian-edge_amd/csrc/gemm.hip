@@ -57,9 +57,7 @@ __device__ __forceinline__ float af_row_mult(const float* amax, int m, int parts
 __device__ __forceinline__ v4i quantize_frag16(const float4 (&f)[4], float a) {
   v4i r;
 #pragma unroll
-  for (int w = 0; w < 4; ++w)
-    r[w] = (quantize_one(f[w].x, a) & 0xFF) | ((quantize_one(f[w].y, a) & 0xFF) << 8) |
-           ((quantize_one(f[w].z, a) & 0xFF) << 16) | ((quantize_one(f[w].w, a) & 0xFF) << 24);
+  for (int w = 0; w < 4; ++w) r[w] = (int)quantize_pack4(f[w], a);
   return r;
 }
 constexpr int kAfRows = 16;  // fp32 A source: one MFMA row tile per workgroup
@@ -168,9 +166,10 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(GemmArgs g, Epilogue e)
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
           const float4 v = raw[i][w];
-          bad |= !isfinite(v.x) || !isfinite(v.y) || !isfinite(v.z) || !isfinite(v.w);
+          bad |= __builtin_isunordered(v.x, v.y) || __builtin_isunordered(v.z, v.w);
           mx = fmaxf(fmaxf(mx, fmaxf(fabsf(v.x), fabsf(v.y))), fmaxf(fabsf(v.z), fabsf(v.w)));
         }
+      bad |= !(mx < INFINITY);
       mx = fmaxf(mx, __shfl_xor(mx, 16));
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       if (lane < kAfRows) sRowMax[wave * kAfRows + lane] = mx;
@@ -179,7 +178,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(GemmArgs g, Epilogue e)
       float rm = 0.0f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) rm = fmaxf(rm, sRowMax[w * kAfRows + (lane & 15)]);
-      a_m = row_multiplier(rm);
+      a_m = g.act > 0.0f ? g.act : row_multiplier(rm);
     }
 #pragma unroll
     for (int i = 0; i < KSW; ++i) {
@@ -209,7 +208,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(GemmArgs g, Epilogue e)
       float rm = 0.0f;
 #pragma unroll
       for (int w = 0; w < NW; ++w) rm = fmaxf(rm, sRowMax[w * kAfRows + m]);
-      am[k] = row_multiplier(rm);
+      am[k] = g.act > 0.0f ? g.act : row_multiplier(rm);
     }
   }
   const int M = RG ? min(Md - r0, kAfRows) : Md;  // this workgroup's rows
@@ -290,7 +289,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(GemmArgs g, Epilogue e)
         }
       } else {
         if (out) out[(int64_t)m * e.ldo + n] = y;
-        if (e.out_i32) e.out_i32[(int64_t)m * e.ldi + n] = iv;
+        if (e.out_i32) e.out_i32[(int64_t)(r0 + m) * e.ldi + n] = iv;
         if (e.out_q) {  // int8 A only (no row offset r0)
           e.out_q[(int64_t)m * e.ldq + n] = (int8_t)quantize_one(y, e.qmult);
           if (n == 0) e.out_qa[m] = e.qmult;
@@ -745,10 +744,15 @@ static hipError_t launch_skinny_k(const GemmArgs& g, const Epilogue& e, hipStrea
 template <int MODE>
 static hipError_t launch_skinny_mode(const GemmArgs& g, const Epilogue& e, hipStream_t s) {
   const int ksteps = g.K >> 6;
-  if (g.Af && !g.Aamax) {  // row maxima found here: the FFN down-projection (K <= 2048)
-    if (MODE != EPI_STORE || ksteps > 32 || g.ldaf % 4 || e.out_i32 || g.M > 65535 * kAfRows)
-      return hipErrorInvalidValue;
-    return launch_skinny_k<MODE, 16, 2, A_F32_MAX>(g, e, s);
+  if (g.Af && !g.Aamax) {  // row maxima found here (or the static multiplier): K <= 2048
+    if constexpr (MODE == EPI_STORE) {
+      if (ksteps > 32 || g.ldaf % 4 || g.M > 65535 * kAfRows) return hipErrorInvalidValue;
+      if (ksteps <= 4) return launch_skinny_k<MODE, 4, 1, A_F32_MAX>(g, e, s);
+      if (ksteps <= 8) return launch_skinny_k<MODE, 8, 1, A_F32_MAX>(g, e, s);
+      if (ksteps <= 16) return launch_skinny_k<MODE, 16, 1, A_F32_MAX>(g, e, s);
+      return launch_skinny_k<MODE, 16, 2, A_F32_MAX>(g, e, s);
+    }
+    return hipErrorInvalidValue;
   }
   if (g.Af) {
     if (MODE != EPI_STORE || ksteps > 8 || !g.Aamax || g.amax_parts < 1 || g.amax_parts > kAfMaxParts ||
@@ -810,6 +814,21 @@ hipError_t launch_vocab_argmax(const GemmArgs& g, const Epilogue& e, hipStream_t
   else
     hipLaunchKernelGGL(kern, grid, block, 0, s, g, e);
   return hipGetLastError();
+}
+
+// Few rows: every workgroup of the skinny kernel quantizes its own 16 rows
+// (a call of 1 x 2048, K = 512, 10.5 -> 7.5 us; 64 x 512, K = 2048, 10.1 ->
+// 8.3).  Above 16 rows a wide output would repeat that in 500 and more
+// workgroups per row group (64 x 32000: 19 us against 7.8 on row tiles).
+static bool linear_f32_skinny(const GemmArgs& g) { return g.M <= kSkinnyRows && (g.M <= kAfRows || g.N < 8192); }
+
+bool linear_f32_fused(const GemmArgs& g, const Epilogue& e) {
+  if (!g.Af || g.Aamax || g.M_dev || e.out_q || g.ldaf % 4 || (uintptr_t)g.Af % 16) return false;
+  return linear_f32_skinny(g) ? g.K <= kSkinnyMaxK : gemm_f32_supported(g, e);
+}
+
+hipError_t launch_linear_f32(const GemmArgs& g, const Epilogue& e, hipStream_t s) {
+  return linear_f32_skinny(g) ? launch_gemm_skinny(g, EPI_STORE, e, s) : launch_gemm_f32(g, e, s);
 }
 
 hipError_t launch_gemm_store(const GemmArgs& g, const Epilogue& e, hipStream_t s) {

@@ -56,6 +56,7 @@ struct GemmArgs {
   int64_t ldaf = 0;
   const float* Aamax = nullptr;
   int amax_parts = 0;
+  float act = 0.0f;  // > 0: the rows' static multiplier instead (no maxima)
   int* err = nullptr;
   // Vocabulary kernel only: with pro.kind == PRO_LN the rows (at most
   // kVocabLnMaxRows, K = 512) are LayerNorm(pro.y + pro.r), built in the
@@ -108,6 +109,15 @@ hipError_t launch_vocab_argmax(const GemmArgs& g, const Epilogue& e, hipStream_t
                                hipEvent_t ev_start = nullptr, hipEvent_t ev_stop = nullptr);
 // LDS-tiled MFMA GEMM for large M (EPI_STORE only); lda a multiple of 16.
 hipError_t launch_gemm_tile(const GemmArgs& g, const Epilogue& e, hipStream_t s);
+// The tile GEMM from fp32 rows Af (quantized in the kernel, each row's own
+// multiplier or the static g.act): K up to 512, 16-byte aligned rows.
+bool gemm_f32_supported(const GemmArgs& g, const Epilogue& e);
+hipError_t launch_gemm_f32(const GemmArgs& g, const Epilogue& e, hipStream_t s);
+// A layer from fp32 rows (g.Af, and g.act or the rows' own multipliers) in one
+// launch; linear_f32_fused says whether the shape takes it, or is faster
+// quantized first.
+bool linear_f32_fused(const GemmArgs& g, const Epilogue& e);
+hipError_t launch_linear_f32(const GemmArgs& g, const Epilogue& e, hipStream_t s);
 // Picks the kernel by M (host-known M only).
 hipError_t launch_gemm_store(const GemmArgs& g, const Epilogue& e, hipStream_t s);
 

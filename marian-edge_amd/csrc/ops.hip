@@ -115,6 +115,49 @@ int vocab_argmax_into(const int8_t* xq, const float* xa, int64_t M, int64_t K, c
   return op_status(launch_argmax_reduce(part, nparts, (int)M, token, s), "vocab_argmax reduce");
 }
 
+// A Q8 layer from fp32 rows x (each row's own multiplier, or the static `act`
+// when positive) or, without x, from quantized rows: one launch where
+// linear_f32_fused says so, else the row quantization into scratch first.
+int linear_op(const float* x, float act, const int8_t* xq, const float* xa, int64_t M, int64_t K, const int8_t* w,
+              const float* w_mult, const float* bias, int64_t N, int relu, int32_t* out_i32, float* out_f32, int* err,
+              hipStream_t s, const char* what) {
+  GemmArgs g;
+  g.lda = K;
+  g.M = (int)M;
+  g.K = (int)K;
+  g.W = w;
+  g.wmult = w_mult;
+  g.bias = bias;
+  g.N = (int)N;
+  Epilogue e;
+  e.out = out_f32;
+  e.ldo = N;
+  e.out_i32 = out_i32;
+  e.ldi = N;
+  e.relu = relu;
+  if (x) {
+    g.Af = x;
+    g.ldaf = K;
+    g.act = act;
+    g.err = err;
+    if (linear_f32_fused(g, e)) return op_status(launch_linear_f32(g, e, s), what);
+    g.Af = nullptr;
+    g.err = nullptr;
+    int8_t* q = (int8_t*)op_scratch(0, (size_t)M * K, s);
+    float* a = (float*)op_scratch(1, (size_t)M * 4, s);
+    if (!q || !a) return op_status(hipErrorOutOfMemory, what);
+    const int rc = op_status(act > 0.0f ? launch_quantize_rows_static(x, K, (int)M, (int)K, act, q, K, a, err, s)
+                                        : launch_quantize_rows(x, K, (int)M, nullptr, (int)K, q, K, a, err, s),
+                             what);
+    if (rc) return rc;
+    xq = q;
+    xa = a;
+  }
+  g.A = xq;
+  g.a = xa;
+  return op_status(launch_gemm_store(g, e, s), what);
+}
+
 bool vocab_args_ok(const int8_t* xq, const float* xa, int64_t M, int64_t K, const int8_t* emb,
                    const float* emb_mult, const float* bias, int64_t V, const int32_t* token) {
   return xq && xa && emb && emb_mult && bias && token && M >= 0 && K > 0 && K % 64 == 0 &&
@@ -143,34 +186,8 @@ int marian_hip_q8_linear(const float* x, const int8_t* xq, const float* xa, int6
       N > INT32_MAX || K > INT32_MAX || (!x && (!xq || !xa)) || (!out_i32 && !out_f32))
     return MARIAN_HIP_ERR_INVALID_INPUT;
   if (M == 0) return MARIAN_HIP_OK;
-  hipStream_t s = (hipStream_t)stream;
-  if (x) {
-    int8_t* q = (int8_t*)op_scratch(0, (size_t)M * K, s);
-    float* a = (float*)op_scratch(1, (size_t)M * 4, s);
-    if (!q || !a) return op_status(hipErrorOutOfMemory, "q8_linear scratch");
-    int rc = op_status(launch_quantize_rows(x, K, (int)M, nullptr, (int)K, q, K, a, err, s),
-                       "q8_linear quantize");
-    if (rc) return rc;
-    xq = q;
-    xa = a;
-  }
-  GemmArgs g;
-  g.A = xq;
-  g.a = xa;
-  g.lda = K;
-  g.M = (int)M;
-  g.K = (int)K;
-  g.W = w;
-  g.wmult = w_mult;
-  g.bias = bias;
-  g.N = (int)N;
-  Epilogue e;
-  e.out = out_f32;
-  e.ldo = N;
-  e.out_i32 = out_i32;
-  e.ldi = N;
-  e.relu = relu;
-  return op_status(launch_gemm_store(g, e, s), "q8_linear gemm");
+  return linear_op(x, 0.0f, xq, xa, M, K, w, w_mult, bias, N, relu, out_i32, out_f32, err, (hipStream_t)stream,
+                   "q8_linear");
 }
 
 int marian_hip_q8_linear_static(const float* x, int64_t M, int64_t K, float act_mult,
@@ -181,30 +198,8 @@ int marian_hip_q8_linear_static(const float* x, int64_t M, int64_t K, float act_
       !std::isfinite(act_mult))
     return MARIAN_HIP_ERR_INVALID_INPUT;
   if (M == 0) return MARIAN_HIP_OK;
-  hipStream_t s = (hipStream_t)stream;
-  int8_t* q = (int8_t*)op_scratch(0, (size_t)M * K, s);
-  float* a = (float*)op_scratch(1, (size_t)M * 4, s);
-  if (!q || !a) return op_status(hipErrorOutOfMemory, "q8_linear_static scratch");
-  int rc = op_status(launch_quantize_rows_static(x, K, (int)M, (int)K, act_mult, q, K, a, err, s),
-                     "q8_linear_static quantize");
-  if (rc) return rc;
-  GemmArgs g;
-  g.A = q;
-  g.a = a;
-  g.lda = K;
-  g.M = (int)M;
-  g.K = (int)K;
-  g.W = w;
-  g.wmult = w_mult;
-  g.bias = bias;
-  g.N = (int)N;
-  Epilogue e;
-  e.out = out_f32;
-  e.ldo = N;
-  e.out_i32 = out_i32;
-  e.ldi = N;
-  e.relu = relu;
-  return op_status(launch_gemm_store(g, e, s), "q8_linear_static gemm");
+  return linear_op(x, act_mult, nullptr, nullptr, M, K, w, w_mult, bias, N, relu, out_i32, out_f32, err,
+                   (hipStream_t)stream, "q8_linear_static");
 }
 
 int marian_hip_ssru_layer_norm(const float* cand, const float* forget, float* state,

@@ -53,6 +53,94 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rows(const void* p, int64
                                            p ? (int)(rows * ld * size) : 0, kRawBufferWord3);
 }
 
+// Dequantizes and stores one wave's blocks of a tile at (m0, n0): rows wr +
+// 32 i, columns wc + 32 k.  sAm: the tile's row multipliers in LDS; ok: this
+// lane's share of them has exponents in recip_exact's range.
+template <int BM, int MB, int NB, bool RELU, bool EXTRA, bool WIDE>
+__device__ __forceinline__ void tile_store(const GemmArgs& g, const Epilogue& e, const v16i (&acc)[MB][NB],
+                                           const float* sAm, const float (&wm)[NB], const float (&bi)[NB], bool ok,
+                                           int m0, int n0, int wr, int wc) {
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+#pragma unroll
+  for (int k = 0; k < NB; ++k) ok &= recip_factor(wm[k]);
+  ok = __all(ok);
+  const float* sm = sAm + wr + 4 * half;
+  const int rows = min(BM, g.M - m0);
+  const uint32_t row0 = (uint32_t)(wr + 4 * half);
+  // Buffer stores whose range ends with the tile's last row drop the rows
+  // past M; a lane past N starts past the range.
+  const __amdgpu_buffer_rsrc_t ro = tile_rows(e.out, (int64_t)m0 * e.ldo, e.ldo, rows, 4);
+  const __amdgpu_buffer_rsrc_t ri = tile_rows(EXTRA ? e.out_i32 : nullptr, (int64_t)m0 * e.ldi, e.ldi, rows, 4);
+  const __amdgpu_buffer_rsrc_t rq = tile_rows(EXTRA ? e.out_q : nullptr, (int64_t)m0 * e.ldq, e.ldq, rows, 1);
+  bool bad = false;
+  int ncol[NB];
+  uint32_t off[NB];
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    ncol[k] = n0 + wc + k * 32 + (lane & 31);
+    off[k] = ncol[k] < g.N ? (row0 * (uint32_t)e.ldo + (uint32_t)ncol[k]) * 4u : 0x80000000u;
+  }
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const float4 a4 = *(const float4*)(sm + i * 32 + 8 * q);
+      const float av[4] = {a4.x, a4.y, a4.z, a4.w};
+      float inv[4][NB];
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int k = 0; k < NB; ++k) inv[r][k] = recip_exact(av[r] * wm[k]);
+      if (!ok) {  // a multiplier outside recip_exact's range: the IEEE quotient
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int k = 0; k < NB; ++k) inv[r][k] = dequant_scale(av[r], wm[k]);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const uint32_t ml = row0 + (uint32_t)(i * 32 + 8 * q + r);  // row of the tile
+#pragma unroll
+        for (int k = 0; k < NB; ++k) {
+          const int32_t iv = acc[i][k][4 * q + r];
+          float y = dequant_apply(iv, inv[r][k], bi[k]);
+          if (RELU) y = y > 0.0f ? y : 0.0f;
+          if constexpr (!EXTRA) {
+            __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ro, off[k], 0, kNt);
+            off[k] += (r == 3 ? 5u : 1u) * (uint32_t)e.ldo * 4u;  // rows 0-3, 8-11, 16-19, 24-27 of each block
+          } else if (WIDE) {  // row strides past the buffer offsets
+            const int64_t m = m0 + (int64_t)ml;
+            if (m < g.M && ncol[k] < g.N) {
+              if (e.out) e.out[m * e.ldo + ncol[k]] = y;
+              if (e.out_i32) e.out_i32[m * e.ldi + ncol[k]] = iv;
+              if (e.out_q) e.out_q[m * e.ldq + ncol[k]] = (int8_t)quantize_one(y, e.qmult);
+              bad |= !isfinite(y);
+            }
+          } else {
+            const bool in = ncol[k] < g.N;
+            const uint32_t n = (uint32_t)ncol[k];
+            if (e.out)
+              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ro,
+                                                    in ? (ml * (uint32_t)e.ldo + n) * 4u : 0x80000000u, 0, kNt);
+            if (e.out_i32)
+              __builtin_amdgcn_raw_buffer_store_b32((uint32_t)iv, ri,
+                                                    in ? (ml * (uint32_t)e.ldi + n) * 4u : 0x80000000u, 0, kNt);
+            if (e.out_q)
+              __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(int8_t)quantize_one(y, e.qmult), rq,
+                                                   in ? ml * (uint32_t)e.ldq + n : 0x80000000u, 0, 0);
+            bad |= in && (int)ml < rows && !isfinite(y);
+          }
+        }
+      }
+    }
+  if constexpr (EXTRA) {
+    if (e.out_q) {
+      if (n0 == 0 && tid < rows) e.out_qa[m0 + tid] = e.qmult;
+      if (__any(bad) && lane == 0 && g.err) *g.err = 1;  // quantizing rejects non-finite input
+    }
+  }
+}
+
 template <int BM, int BN, int WM, int WN, int PF, bool RELU, bool EXTRA, bool WIDE>
 __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(BM > 128 ? 2 : WM * WN / 2)))
 void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
@@ -177,91 +265,146 @@ void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
         }
       }
     }
-    // ---- epilogue ----
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < BM; i += 64) ok &= recip_factor(sAm[tpar][i + lane]);
-#pragma unroll
-    for (int k = 0; k < NB; ++k) ok &= recip_factor(wm[k]);
-    ok = __all(ok);
-    const float* sm = sAm[tpar] + wr + 4 * half;
-    const int rows = min(BM, M - m0);
-    const uint32_t row0 = (uint32_t)(wr + 4 * half);
-    // Buffer stores whose range ends with the tile's last row drop the rows
-    // past M; a lane past N starts past the range.
-    const __amdgpu_buffer_rsrc_t ro = tile_rows(e.out, (int64_t)m0 * e.ldo, e.ldo, rows, 4);
-    const __amdgpu_buffer_rsrc_t ri = tile_rows(EXTRA ? e.out_i32 : nullptr, (int64_t)m0 * e.ldi, e.ldi, rows, 4);
-    const __amdgpu_buffer_rsrc_t rq = tile_rows(EXTRA ? e.out_q : nullptr, (int64_t)m0 * e.ldq, e.ldq, rows, 1);
-    bool bad = false;
-    int ncol[NB];
-    uint32_t off[NB];
-#pragma unroll
-    for (int k = 0; k < NB; ++k) {
-      ncol[k] = n0 + wc + k * 32 + (lane & 31);
-      off[k] = ncol[k] < N ? (row0 * (uint32_t)e.ldo + (uint32_t)ncol[k]) * 4u : 0x80000000u;
-    }
-#pragma unroll
-    for (int i = 0; i < MB; ++i)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const float4 a4 = *(const float4*)(sm + i * 32 + 8 * q);
-        const float av[4] = {a4.x, a4.y, a4.z, a4.w};
-        float inv[4][NB];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int k = 0; k < NB; ++k) inv[r][k] = recip_exact(av[r] * wm[k]);
-        if (!ok) {  // a multiplier outside recip_exact's range: the IEEE quotient
-#pragma unroll
-          for (int r = 0; r < 4; ++r)
-#pragma unroll
-            for (int k = 0; k < NB; ++k) inv[r][k] = dequant_scale(av[r], wm[k]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const uint32_t ml = row0 + (uint32_t)(i * 32 + 8 * q + r);  // row of the tile
-#pragma unroll
-          for (int k = 0; k < NB; ++k) {
-            const int32_t iv = acc[i][k][4 * q + r];
-            float y = dequant_apply(iv, inv[r][k], bi[k]);
-            if (RELU) y = y > 0.0f ? y : 0.0f;
-            if constexpr (!EXTRA) {
-              __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ro, off[k], 0, kNt);
-              off[k] += (r == 3 ? 5u : 1u) * (uint32_t)e.ldo * 4u;  // rows 0-3, 8-11, 16-19, 24-27 of each block
-            } else if (WIDE) {  // row strides past the buffer offsets
-              const int64_t m = m0 + (int64_t)ml;
-              if (m < M && ncol[k] < N) {
-                if (e.out) e.out[m * e.ldo + ncol[k]] = y;
-                if (e.out_i32) e.out_i32[m * e.ldi + ncol[k]] = iv;
-                if (e.out_q) e.out_q[m * e.ldq + ncol[k]] = (int8_t)quantize_one(y, e.qmult);
-                bad |= !isfinite(y);
-              }
-            } else {
-              const bool in = ncol[k] < N;
-              const uint32_t n = (uint32_t)ncol[k];
-              if (e.out)
-                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(y), ro,
-                                                      in ? (ml * (uint32_t)e.ldo + n) * 4u : 0x80000000u, 0, kNt);
-              if (e.out_i32)
-                __builtin_amdgcn_raw_buffer_store_b32((uint32_t)iv, ri,
-                                                      in ? (ml * (uint32_t)e.ldi + n) * 4u : 0x80000000u, 0, kNt);
-              if (e.out_q)
-                __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(int8_t)quantize_one(y, e.qmult), rq,
-                                                     in ? ml * (uint32_t)e.ldq + n : 0x80000000u, 0, 0);
-              bad |= in && (int)ml < rows && !isfinite(y);
-            }
-          }
-        }
-      }
-    if constexpr (EXTRA) {
-      if (e.out_q) {
-        if (n0 == 0 && tid < rows) e.out_qa[m0 + tid] = e.qmult;
-        if (__any(bad) && lane == 0 && g.err) *g.err = 1;  // quantizing rejects non-finite input
-      }
-    }
+    tile_store<BM, MB, NB, RELU, EXTRA, WIDE>(g, e, acc, sAm[tpar], wm, bi, ok, m0, n0, wr, wc);
     m0 = m1;
     n0 = n1;
   }
+}
+
+// ---------------------------------------------------------------------------
+// The same product from fp32 rows: a workgroup quantizes its 64 rows itself
+// (row multiplier 127 / max|x|, or the static one in g.act) into LDS for the
+// whole K (at most 512), then streams the weights past them, so the layer is
+// one launch.  Each row is quantized once per column tile, which costs less
+// than the launch and the pass over memory it replaces while the shape is at
+// most one round of workgroups (gemm_f32_supported).  A serial chain of one
+// tile bounds it: the rows' round trip, 1.3 us of quantizing (39 instructions
+// a row and wave: a row on 16 lanes needs four lane moves for its maximum and
+// shares one division, against 90 with a row per wave), the K loop, the
+// stores.  1459 x 512, K = 512: 10.0 us a call in two launches, 7.4 in one.
+// ---------------------------------------------------------------------------
+constexpr int kF32MaxK = 512;
+constexpr int kF32Rows = 64;
+
+template <int BN, int WM, int WN, bool RELU, bool EXTRA>
+__global__ __launch_bounds__(WM * WN * 64) void k_gemm_tile_f32(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
+  constexpr int BM = kF32Rows, NW = WM * WN, NT = NW * 64;
+  constexpr int MB = BM / WM / 32, NB = BN / WN / 32, BP = BN * 8 / NT, PF = 2;
+  __shared__ __attribute__((aligned(16))) int8_t sA[BM * kF32MaxK];  // [128-byte chunk][row][piece ^ row % 8]
+  __shared__ __attribute__((aligned(16))) int8_t sB[2][BN * kTileKC];
+  __shared__ float sAm[BM];
+  const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr = wave / WN * (BM / WM), wc = wave % WN * (BN / WN);
+  const int M = g.M, N = g.N, K = g.K;
+  const int xcd = blockIdx.x & 7;
+  const int tile = (int)((int64_t)xcd * tiles >> 3) + (blockIdx.x >> 3);
+  if (tile >= (int)((int64_t)(xcd + 1) * tiles >> 3)) return;  // the whole workgroup
+  const int m0 = tile / tiles_n * BM, n0 = tile % tiles_n * BN;
+  const int nslot = (K + 2 * kTileKC - 1) / (2 * kTileKC) * 2;  // 2 or 4 chunks
+
+  const int8_t* pb[BP];
+  v4i rb[PF][BP];
+  const int kp = (tid & 7) * 16;
+  auto gload = [&](int c, v4i (&xb)[BP]) {
+    const int col = min(c * kTileKC + kp, K - 16);
+#pragma unroll
+    for (int i = 0; i < BP; ++i) xb[i] = *(const v4i*)(pb[i] + col);
+  };
+#pragma unroll
+  for (int i = 0; i < BP; ++i) pb[i] = g.W + (int64_t)min(n0 + ((tid + i * NT) >> 3), N - 1) * K;
+
+  // ---- the rows: a wave takes four at a time, 16 lanes each; lane l of them
+  // holds columns 4l + 64j ----
+  constexpr int RW = BM / NW, G = RW / 4;  // rows per wave, groups of four
+  const int kj = K >> 6;                   // live j
+  const int c4 = 4 * (lane & 15);
+  float4 v[G][8];
+#pragma unroll
+  for (int t = 0; t < G; ++t) {
+    const float* xr = g.Af + (int64_t)min(m0 + wave * RW + 4 * t + (lane >> 4), M - 1) * g.ldaf + c4;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[t][j] = *(const float4*)(xr + 64 * min(j, kj - 1));  // past K: the last again
+  }
+#pragma unroll
+  for (int u = 0; u < PF; ++u) gload(u, rb[u]);  // the first weights arrive under the quantization
+  bool bad = false;
+#pragma unroll
+  for (int t = 0; t < G; ++t) {
+    const int row = wave * RW + 4 * t + (lane >> 4);
+    float mx = 0.0f;
+    bool nan = false;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const float4 x = v[t][j];
+      mx = fmaxf(fmaxf(mx, fmaxf(fabsf(x.x), fabsf(x.y))), fmaxf(fabsf(x.z), fabsf(x.w)));
+      nan |= __builtin_isunordered(x.x, x.y) || __builtin_isunordered(x.z, x.w);
+    }
+    bad |= (nan || !(mx < INFINITY)) && m0 + row < M;
+    mx = fmaxf(mx, __int_as_float(dpp_mov<0xB1>(__float_as_int(mx))));   // over the row's 16 lanes
+    mx = fmaxf(mx, __int_as_float(dpp_mov<0x4E>(__float_as_int(mx))));
+    mx = fmaxf(mx, __int_as_float(dpp_mov<0x124>(__float_as_int(mx))));
+    mx = fmaxf(mx, __int_as_float(dpp_mov<0x128>(__float_as_int(mx))));
+    const float a = g.act > 0.0f ? g.act : row_multiplier(mx);
+    if ((lane & 15) == 0) sAm[row] = a;
+    int8_t* ar = sA + row * kTileKC + (c4 & 15);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int c = c4 + 64 * j;
+      if (j < 2 * nslot)  // uniform; a last chunk past K holds zeros
+        *(uint32_t*)(ar + (j >> 1) * (BM * kTileKC) + ((((c >> 4) & 7) ^ (row & 7)) << 4)) =
+            j < kj ? quantize_pack4(v[t][j], a) : 0u;
+    }
+  }
+  if (__any(bad) && lane == 0 && g.err) *g.err = 1;
+
+  // ---- the weights past them ----
+  v16i acc[MB][NB];
+#pragma unroll
+  for (int i = 0; i < MB; ++i)
+#pragma unroll
+    for (int k = 0; k < NB; ++k)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][k][r] = 0;
+  float wm[NB], bi[NB];
+#pragma unroll
+  for (int k = 0; k < NB; ++k) {
+    const int n = min(n0 + wc + k * 32 + (lane & 31), N - 1);
+    wm[k] = g.wmult[n];
+    bi[k] = g.bias[n];
+  }
+  for (int c0 = 0; c0 < nslot; c0 += PF) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+#pragma unroll
+      for (int i = 0; i < BP; ++i) {
+        const int c = tid + i * NT, row = c >> 3;
+        *(v4i*)(sB[u & 1] + row * kTileKC + (((c & 7) ^ (row & 7)) << 4)) = rb[u][i];
+      }
+      gload(c0 + PF + u, rb[u]);  // past K: the last pieces again, unused
+      wg_lds_barrier();
+      const int8_t* la = sA + (c0 + u) * (BM * kTileKC) + (wr + (lane & 31)) * kTileKC;
+      const int8_t* lb = sB[u & 1] + (wc + (lane & 31)) * kTileKC;
+#pragma unroll
+      for (int ks = 0; ks < kTileKC / 32; ++ks) {
+        const int at = ((2 * ks + half) ^ (lane & 7)) << 4;
+        v4i fa[MB], fb[NB];
+#pragma unroll
+        for (int i = 0; i < MB; ++i) fa[i] = *(const v4i*)(la + i * 32 * kTileKC + at);
+#pragma unroll
+        for (int k = 0; k < NB; ++k) fb[k] = *(const v4i*)(lb + k * 32 * kTileKC + at);
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+          for (int k = 0; k < NB; ++k)
+            acc[i][k] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i], fb[k], acc[i][k], 0, 0, 0);
+      }
+    }
+  }
+  tile_store<BM, MB, NB, RELU, EXTRA, false>(g, e, acc, sAm, wm, bi, recip_factor(sAm[lane]), m0, n0, wr, wc);
 }
 
 template <int BM, int BN, int WM, int WN, int PF, bool WIDE = false>
@@ -273,6 +416,17 @@ hipError_t launch_tile(const GemmArgs& g, const Epilogue& e, int max_wgs, hipStr
   auto kern = e.relu ? (extra ? k_gemm_tile<BM, BN, WM, WN, PF, true, true, WIDE> : k_gemm_tile<BM, BN, WM, WN, PF, true, WIDE, WIDE>)
                      : (extra ? k_gemm_tile<BM, BN, WM, WN, PF, false, true, WIDE> : k_gemm_tile<BM, BN, WM, WN, PF, false, WIDE, WIDE>);
   hipLaunchKernelGGL(kern, dim3(grid), dim3(WM * WN * 64), 0, s, g, e, (int)tiles_n, (int)tiles);
+  return hipGetLastError();
+}
+
+template <int BN, int WM, int WN>
+hipError_t launch_tile_f32(const GemmArgs& g, const Epilogue& e, hipStream_t s) {
+  const int64_t tiles_n = (g.N + BN - 1) / BN, tiles = (g.M + kF32Rows - 1) / kF32Rows * tiles_n;
+  if (tiles > (1 << 30)) return hipErrorInvalidValue;
+  const bool extra = e.out_i32 || e.out_q || !e.out;
+  auto kern = e.relu ? (extra ? k_gemm_tile_f32<BN, WM, WN, true, true> : k_gemm_tile_f32<BN, WM, WN, true, false>)
+                     : (extra ? k_gemm_tile_f32<BN, WM, WN, false, true> : k_gemm_tile_f32<BN, WM, WN, false, false>);
+  hipLaunchKernelGGL(kern, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(WM * WN * 64), 0, s, g, e, (int)tiles_n, (int)tiles);
   return hipGetLastError();
 }
 
@@ -298,6 +452,28 @@ hipError_t launch_gemm_tile(const GemmArgs& g, const Epilogue& e, hipStream_t s)
   if (tiles(256, 128) >= 2048) return launch_tile<256, 128, 4, 2, 2>(g, e, 256, s);
   if (tiles(128, 128) >= 224) return launch_tile<128, 128, 2, 4, 2>(g, e, 1 << 30, s);
   return launch_tile<64, 64, 2, 2, 2>(g, e, 1024, s);
+}
+
+static int64_t f32_tiles(const GemmArgs& g, int bn) {
+  return (int64_t)((g.M + kF32Rows - 1) / kF32Rows) * ((g.N + bn - 1) / bn);
+}
+
+bool gemm_f32_supported(const GemmArgs& g, const Epilogue& e) {
+  const int64_t ld = std::max(std::max(e.out ? e.ldo : 0, e.out_i32 ? e.ldi : 0), e.out_q ? e.ldq : 0);
+  // More than a round of 256-column tiles is faster quantized first, as one
+  // pass: 2500 x 2048 (320 tiles) 15.4 us a call against 12.7 in two launches,
+  // 7405 x 512 (232) 8.9 against 12.6.
+  return g.Af && g.K <= kF32MaxK && g.ldaf % 4 == 0 && (uintptr_t)g.Af % 16 == 0 && ld < (1 << 20) &&
+         f32_tiles(g, 256) <= 256;
+}
+
+hipError_t launch_gemm_f32(const GemmArgs& g, const Epilogue& e, hipStream_t s) {
+  if (g.K <= 0 || g.K % 64 || g.N <= 0 || g.M_dev || !gemm_f32_supported(g, e)) return hipErrorInvalidValue;
+  if (g.M <= 0) return hipSuccess;
+  // One round of workgroups either way: 128 columns a tile while that fits the
+  // 256 CUs (1459 x 512: 7.9 us, 8.5 with 256 columns), else 256 columns on 16
+  // waves (1459 x 2048: 9.8 us, 11.0 with 128).
+  return f32_tiles(g, 128) <= 256 ? launch_tile_f32<128, 2, 4>(g, e, s) : launch_tile_f32<256, 2, 8>(g, e, s);
 }
 
 }  // namespace mh

@@ -113,6 +113,62 @@ def test_q8_linear_tile_sizes(dev, M, K, N):
             assert np.array_equal(df.host().view(np.uint32), want.view(np.uint32)), f"both relu={relu}"
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (1, 64, 33), (16, 448, 100), (17, 512, 96), (64, 1024, 1030), (61, 1536, 384), (3, 2048, 70),  # 16-row groups
+    (17, 512, 8200), (64, 64, 9000), (65, 192, 127), (129, 512, 1000),  # row tiles, 128 columns
+    (1100, 320, 2300),                                                  # row tiles, 256 columns
+    (65, 576, 64), (5000, 512, 2048),                                   # quantized first
+])
+@pytest.mark.parametrize("act", [0.0, 31.75])
+def test_q8_linear_from_fp32_rows(dev, M, K, N, act):
+    """The layer from fp32 rows (their own multipliers, or a static one that clamps the
+    largest values) equals the row quantization followed by the layer on its int8 rows,
+    bit for bit: zero rows, a row whose multiplier overflows to infinity, halfway values,
+    and the error flag of a non-finite value."""
+    print(f"q8_linear fp32 rows M={M} K={K} N={N} act={act}", flush=True)
+    rng = np.random.default_rng(M + K + N)
+    x = (rng.standard_normal((M, K)) * rng.uniform(0.1, 4, size=(M, 1))).astype(np.float32)
+    x[0, :8] = [0.5, 1.5, -0.5, -1.5, 2.5, -2.5, 0.0, -0.0]
+    if M > 2:
+        x[1] = 0.0
+        x[2] = 0.0
+        x[2, ::3] = np.float32(1e-38)  # 127 / 1e-38 overflows
+    w = rng.integers(-127, 128, size=(N, K)).astype(np.int8)
+    mult = rng.uniform(50, 100, size=N).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    D = dev.DeviceArray
+    dw, dm, db = (D.from_host(v) for v in (w, mult, bias))
+    # The static multiplier on the host, the rows' own by the quantization kernel.
+    dx = D.from_host(x)
+    if act:
+        dq = D.from_host(np.clip(np.rint(x * np.float32(act)), -127, 127).astype(np.int8))
+        da = D.from_host(np.full(M, act, np.float32))
+    else:
+        dq, da = D.zeros((M, K), np.int8), D.zeros(M, np.float32)
+        dev.quantize_rows(dx, dq, da)
+    for bad in (False, True):
+        if bad:
+            x[M - 1, K - 1] = np.nan if M % 2 else np.inf
+            dx = D.from_host(x)
+        for relu, ints in ((False, True), (True, False)):
+            wi, gi = (D.zeros((M, N), np.int32) if ints else None for _ in range(2))
+            wf, gf = (D.zeros((M, N), np.float32) for _ in range(2))
+            err = D.zeros(1, np.int32)
+            if act:
+                dev.q8_linear_static(dx, act, dw, dm, db, gi, gf, relu=relu, err=err)
+            else:
+                dev.q8_linear(dx, dw, dm, db, gi, gf, relu=relu, err=err)
+            dev.synchronize()
+            assert err.host()[0] == int(bad)
+            if bad:
+                continue
+            dev.q8_linear(None, dw, dm, db, wi, wf, relu=relu, xq=dq, xa=da)
+            dev.synchronize()
+            assert np.array_equal(gf.host().view(np.uint32), wf.host().view(np.uint32))
+            if ints:
+                assert np.array_equal(gi.host(), wi.host())
+
+
 def test_q8_linear_on_two_streams_at_once(pkg, orc, dev):
     """The op-level entry points keep their intermediate buffers (here the
     quantized activations of an fp32 input) per (device, stream): two streams
