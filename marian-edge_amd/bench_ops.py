@@ -309,7 +309,7 @@ def step_breakdown(trace_csv: str, steps_per_batch: int, batches: int, rows_at: 
         if k[0].startswith("k_finalize"):
             steps.append(cur)
             cur = []
-    enc = ("k_gemm_tile", "k_attn_tiles", "k_seq_tiles", "k_embed", "k_quantize_rows_v4<2>")
+    enc = ("k_gemm_tile", "k_attn_seq", "k_embed", "k_quantize_rows_v4<2>")
     groups = [(1, 1), (2, 4), (5, 8), (9, 16), (17, 32), (33, 64), (65, 128), (129, 256), (257, 4096)]
     agg: dict = {}
     for b in range(first_batch, first_batch + batches):

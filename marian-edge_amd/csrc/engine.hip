@@ -129,7 +129,7 @@ int model_fail(const char* fmt, ...) {
 enum Buf {
   B_META, B_DMETA, B_X0, B_X1, B_XQ, B_XA, B_QKV, B_ATT, B_OQ, B_OA, B_Y, B_H, B_HQ, B_HA, B_CKV,
   B_KC, B_VC, B_DX0, B_DX1, B_DXQ, B_DXA, B_DQ, B_DATT, B_DAMAX, B_DY, B_DH, B_DHQ, B_DHA,
-  B_PART, B_OUT, B_COUNT, B_HIST, B_TILES, B_STATE, B_DUF, B_COUNT_,
+  B_PART, B_OUT, B_COUNT, B_HIST, B_STATE, B_DUF, B_COUNT_,
   // allocated only by marian_hip_translate_probe: the probed step's logits
   // and its active-row order
   B_PLOG = B_COUNT_, B_PSLOT, B_ALL_
@@ -827,8 +827,7 @@ struct CallBufs {
   float *DX0, *DX1, *DXA, *DQ, *DATT, *DAMAX, *DY, *DH, *DHA;
   uint64_t* PART;
   int32_t* OUT;
-  uint32_t *COUNT, *HIST, *TILES;
-  int tiles_cap = 0;
+  uint32_t *COUNT, *HIST;
 };
 
 // Grows the engine's capacities to `cs` (with headroom) and fetches every
@@ -904,8 +903,6 @@ int plan_buffers(marian_hip_engine* E, const CallShape& cs, MetaLayout& L, CallB
   b.OUT = (int32_t*)E->get(B_OUT, 4 * CR);
   b.COUNT = (uint32_t*)E->get(B_COUNT, 4 * R);
   b.HIST = (uint32_t*)E->get(B_HIST, 4 * E->hcap);
-  b.tiles_cap = seq_tiles_bound((int)T, (int)B);
-  b.TILES = (uint32_t*)E->get(B_TILES, 4 * (1 + 2 * (size_t)b.tiles_cap));
   for (int i = 0; i < B_COUNT_; ++i)
     if (!E->buf[i]) return E->fail(MARIAN_HIP_ERR_DEVICE, "device allocation failed");
   if (!E->host(marian_hip_engine::H_META, L.meta_bytes) || !E->host(marian_hip_engine::H_DMETA, L.dmeta_bytes) ||
@@ -958,7 +955,6 @@ struct Translation {
   uint32_t gen_limit = 0;
   size_t cache_rows = 1;
   int n_active0 = 0, nparts = 0;
-  bool tiled = false;
   bool fast = false;  // MARIAN_HIP_FLAG_FAST_REDUCTIONS: the decoder's sums in the tree order
   MetaLayout L{};
   CallBufs b{};
@@ -1094,7 +1090,6 @@ int Translation::prepare() {
   rm.srcn = (int32_t*)(b.ddec + L.o_rsrcn);
   rm.prev = (int32_t*)(b.ddec + L.o_rprev);
   rm.limit = (uint32_t*)(b.ddec + L.o_rlim);
-  tiled = bs.Lmax <= 256;
   return MARIAN_HIP_OK;
 }
 
@@ -1135,8 +1130,6 @@ hipError_t Translation::encode() {
     ea.err = E->err_flag;
     MH_TRY(launch_embed(ea, s));
   }
-  // Query tiles of the packed sentences for the encoder's self-attention.
-  if (tiled) MH_TRY(launch_seq_tiles(d_cu, Bi, b.TILES, b.tiles_cap, s));
   auto gemm = [&](const int8_t* A, const float* a, int M, const Lin& L, float* out, int relu,
                   int64_t ldo = 0, int8_t* q = nullptr, float* qa = nullptr, float qmult = 0.0f) {
     GemmArgs g;
@@ -1190,10 +1183,7 @@ hipError_t Translation::encode() {
     aa.seq_of_row = d_seq;
     aa.cu = d_cu;
     aa.max_keys = (int)bs.Lmax;
-    if (tiled) {
-      aa.tiles = b.TILES;
-      aa.tiles_cap = b.tiles_cap;
-    }
+    aa.n_seqs = Bi;
     aa.out = b.ATT;
     aa.ldo = d;
     aa.err = E->err_flag;

@@ -319,19 +319,19 @@ struct AttnArgs {
   int64_t ldqout = 0;
   float qmult = 0.0f;
   float* qa = nullptr;
-  // ATT_SEQ with max_keys <= 256: the query-tile list written by
-  // launch_seq_tiles (tiles_cap = its bound) selects the tiled kernel (no amax).
-  const uint32_t* tiles = nullptr;
-  int tiles_cap = 0;
+  // ATT_SEQ: the sequences in cu when the query rows are their key rows (row i
+  // of sequence s lies in [cu[s], cu[s+1])); with max_keys <= kSeqMaxKeys they
+  // run on launch_attention_seq's kernel (no amax).
+  int n_seqs = 0;
   int fast = 0;  // ATT_CROSS / ATT_SELF: the softmax denominator in the fast-reduction tree order
 };
 // ev_start / ev_stop as in launch_vocab_argmax (single-wave kernel only).
 hipError_t launch_attention(const AttnArgs& a, hipStream_t s, hipEvent_t ev_start = nullptr,
                             hipEvent_t ev_stop = nullptr);
-// Query tiles of packed sequences cu[0..nseq] for the tiled ATT_SEQ kernel:
-// at most seq_tiles_bound(rows, nseq) entries; tiles needs 1 + 2 * cap words.
-int seq_tiles_bound(int rows, int nseq);
-hipError_t launch_seq_tiles(const uint32_t* cu, int nseq, uint32_t* tiles, int cap, hipStream_t s);
+// Packed self-attention (a.n_seqs > 0) over at most kSeqMaxKeys keys, one
+// workgroup per 64 (few rows: 16) queries of a (sequence, head).
+constexpr int kSeqMaxKeys = 512;
+hipError_t launch_attention_seq(const AttnArgs& a, hipStream_t s);
 
 // Decode attention block (one launch per attention sublayer on steps with few
 // rows): per (row, head) it builds the row's input with `pro` (PRO_LN, or

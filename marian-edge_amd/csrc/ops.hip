@@ -35,8 +35,8 @@ int op_status(hipError_t e, const char* what) {
 // Sets live until the process ends (a stream that is destroyed leaves its
 // set behind).
 struct OpScratch {
-  void* p[4] = {nullptr, nullptr, nullptr, nullptr};
-  size_t cap[4] = {0, 0, 0, 0};
+  void* p[3] = {nullptr, nullptr, nullptr};
+  size_t cap[3] = {0, 0, 0};
 };
 std::mutex g_scratch_mu;
 std::map<std::pair<int, uintptr_t>, OpScratch> g_scratch;
@@ -249,17 +249,7 @@ int marian_hip_attention(const void* q, int64_t ldq, const void* k, const void* 
   a.out = out;
   a.ldo = ldo;
   a.max_keys = (int)max_keys;
-  if (n_seqs > 0 && rows > 0 && max_keys <= 256) {
-    // Packed self-attention: the query-tile list first (library scratch).
-    const int cap = seq_tiles_bound((int)rows, (int)n_seqs);
-    uint32_t* tiles = (uint32_t*)op_scratch(3, (1 + 2 * (size_t)cap) * 4, (hipStream_t)stream);
-    if (!tiles) return op_status(hipErrorOutOfMemory, "attention scratch");
-    const int rc = op_status(launch_seq_tiles(cu_k, (int)n_seqs, tiles, cap, (hipStream_t)stream),
-                             "attention tiles");
-    if (rc != MARIAN_HIP_OK) return rc;
-    a.tiles = tiles;
-    a.tiles_cap = cap;
-  }
+  a.n_seqs = (int)n_seqs;
   return op_status(launch_attention(a, (hipStream_t)stream), "attention");
 }
 

@@ -43,22 +43,15 @@
 
 namespace mh {
 
-// `tab` holds the 32 entries of MH_EXP2_TABLE_32 (in LDS or constant memory
-// on the device).
-MH_HOST_DEVICE inline float ref_expf(float x, const uint64_t* tab) {
+// The table-driven part: exp(x) wherever neither overflow nor underflow cuts it
+// off (NaN gives NaN).  `tab` holds the 32 entries of MH_EXP2_TABLE_32 (in LDS
+// or constant memory on the device).
+MH_HOST_DEVICE inline float ref_expf_core(float x, const uint64_t* tab) {
   constexpr double kInvLn2N = 0x1.71547652b82fep+0 * 32;
   constexpr double kShift = 0x1.8p+52;
   constexpr double kC0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32;
   constexpr double kC1 = 0x1.ebfce50fac4f3p-3 / 32 / 32;
   constexpr double kC2 = 0x1.62e42ff0c52d6p-1 / 32;
-  const uint32_t ux = __builtin_bit_cast(uint32_t, x);
-  const uint32_t abstop = (ux >> 20) & 0x7ffu;
-  if (abstop >= 0x42bu) {                      // |x| >= 88 or x is NaN
-    if (ux == 0xff800000u) return 0.0f;        // exp(-inf)
-    if (abstop >= 0x7f8u) return x + x;        // +inf, NaN
-    if (x > 0x1.62e42ep6f) return __builtin_huge_valf();  // overflow
-    if (x < -0x1.9fe368p6f) return 0.0f;       // underflow
-  }
   const double xd = (double)x;
   double kd = __builtin_fma(kInvLn2N, xd, kShift);
   const uint64_t ki = __builtin_bit_cast(uint64_t, kd);
@@ -72,6 +65,24 @@ MH_HOST_DEVICE inline float ref_expf(float x, const uint64_t* tab) {
   y = __builtin_fma(z, r2, y);
   y = y * s;
   return (float)y;
+}
+
+MH_HOST_DEVICE inline float ref_expf(float x, const uint64_t* tab) {
+  const uint32_t ux = __builtin_bit_cast(uint32_t, x);
+  const uint32_t abstop = (ux >> 20) & 0x7ffu;
+  if (abstop >= 0x42bu) {                      // |x| >= 88 or x is NaN
+    if (ux == 0xff800000u) return 0.0f;        // exp(-inf)
+    if (abstop >= 0x7f8u) return x + x;        // +inf, NaN
+    if (x > 0x1.62e42ep6f) return __builtin_huge_valf();  // overflow
+    if (x < -0x1.9fe368p6f) return 0.0f;       // underflow
+  }
+  return ref_expf_core(x, tab);
+}
+
+// The same for x <= 0 or NaN, without branches.
+MH_HOST_DEVICE inline float ref_expf_nonpos(float x, const uint64_t* tab) {
+  const float y = ref_expf_core(x, tab);
+  return x < -0x1.9fe368p6f ? 0.0f : y;
 }
 
 }  // namespace mh

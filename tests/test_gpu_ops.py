@@ -459,6 +459,57 @@ def test_attention_edges(pkg, orc, dev):
     _attention_case(pkg, orc, dev, q, k, v, cu, 8, False)
 
 
+@pytest.mark.parametrize("heads,head_dim,bf16,lens", [
+    # every class of sequence length (up to 16, 32 and 64 m rows) and its edges, few rows and many
+    (8, 64, False, [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 96, 97, 128, 129, 192, 193, 255, 256, 7]),
+    (8, 64, False, [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 96, 97, 128, 129, 192, 193, 255, 256, 7] * 3),
+    (8, 48, True, [256, 1, 33, 100, 16, 32]),
+    (8, 48, True, [256, 1, 33, 100, 16, 32] * 12),
+    # heads that leave a shared workgroup's last places empty
+    (3, 64, True, [5, 16, 20, 32, 40, 130] * 50),
+    (5, 48, False, [16, 17, 64, 65] * 50),
+    # 257 to 512 keys: the variants that hold 512 scores a query
+    (4, 64, False, [257, 320, 321, 511, 512, 3, 30]),
+    (4, 64, False, [257, 320, 321, 511, 512, 3, 30] * 3),
+    (4, 48, True, [400, 17, 449] * 8),
+    # more sequences than one pass of the lookup, and more than it takes
+    (4, 64, False, [1 + (7 * i) % 50 for i in range(600)]),
+    (2, 64, False, [1 + (11 * i) % 70 for i in range(1030)]),
+])
+def test_packed_attention_units(pkg, orc, dev, heads, head_dim, bf16, lens):
+    """Packed self-attention against the oracle, bit for bit, with row strides
+    wider than the rows and one sequence holding infinite and NaN keys."""
+    print(f"packed attention heads={heads} head_dim={head_dim} bf16={bf16} n={len(lens)}", flush=True)
+    rng = np.random.default_rng(41)
+    lens = np.array(lens, np.int64)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    T, d = int(cu[-1]), heads * head_dim
+    ld = (d + 15) // 8 * 8
+    wide = [rng.standard_normal((T, ld)).astype(np.float32) for _ in range(3)]
+    wide[0][:: 3] *= 40.0  # scores far apart: exponentials down to denormals and zero
+    r = int(cu[1])
+    wide[1][r, 0], wide[1][r, head_dim - 1] = np.inf, np.nan
+    if bf16:
+        dev_in = [dev.DeviceArray.from_host(pkg.synthetic.bf16_round(x)) for x in wide]
+        wide = [pkg.synthetic.bf16_to_f32(pkg.synthetic.bf16_round(x)) for x in wide]
+    else:
+        dev_in = [dev.DeviceArray.from_host(x) for x in wide]
+    q, k, v = (np.ascontiguousarray(x[:, :d]) for x in wide)
+    with np.errstate(all="ignore"):
+        ref = orc.attention(q, k, v, cu, cu, heads)
+    seq = np.repeat(np.arange(len(lens), dtype=np.int32), lens)
+    out = dev.DeviceArray.zeros((T, d + 1), np.float32)
+    dev.attention(*dev_in, dev.DeviceArray.from_host(seq), dev.DeviceArray.from_host(cu), out, heads=heads,
+                  max_keys=int(lens.max()), bf16=bf16, head_dim=head_dim)
+    dev.synchronize()
+    got = out.host()
+    assert np.all(got[:, d] == 0.0)
+    got = np.ascontiguousarray(got[:, :d])
+    nan = np.isnan(ref)
+    assert np.array_equal(nan, np.isnan(got))
+    assert np.array_equal(np.where(nan, 0, got).view(np.uint32), np.where(nan, 0, ref).view(np.uint32))
+
+
 @pytest.mark.parametrize("M", [1, 64, 130])
 def test_vocab_argmax_matches_oracle(pkg, orc, dev, full_model, M):
     """Up to 64 rows one row group; 130 rows run three 64-row groups side
