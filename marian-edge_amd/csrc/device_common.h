@@ -112,6 +112,14 @@ __device__ __forceinline__ float wave_max(float p) {
   return fmaxf(fmaxf(r0, r1), fmaxf(r2, r3));
 }
 
+// Maximum over each 16-lane row of the wave (every lane returns its row's).
+__device__ __forceinline__ uint32_t row16_max(uint32_t p) {
+  p = max(p, (uint32_t)dpp_mov<0xB1>((int)p));   // quad_perm [1,0,3,2]
+  p = max(p, (uint32_t)dpp_mov<0x4E>((int)p));   // quad_perm [2,3,0,1]
+  p = max(p, (uint32_t)dpp_mov<0x124>((int)p));  // row_ror:4
+  return max(p, (uint32_t)dpp_mov<0x128>((int)p));  // row_ror:8
+}
+
 // Maximum over each 32-lane half of the wave (every lane returns its half's):
 // the row maxima by DPP, then rows 0-1 and 2-3 paired by a lane swap.
 __device__ __forceinline__ float half_wave_max(float p) {
@@ -500,11 +508,13 @@ __device__ __forceinline__ v4i frag_load(const int8_t* Wf, int tile, int ksteps,
 // The scan starts from -inf at the first candidate and never takes a NaN, so
 // NaN ranks with -inf (a row of only -inf/NaN logits yields its first
 // candidate); -0.0 equals +0.0 under '>', so it is folded into +0.0.
-__device__ __forceinline__ uint64_t argmax_key(float v, uint32_t id) {
+__device__ __forceinline__ uint32_t argmax_order(float v) {
   v = (v != v) ? -INFINITY : v + 0.0f;
   const uint32_t b = __float_as_uint(v);
-  const uint32_t k = (b & 0x80000000u) ? ~b : (b | 0x80000000u);
-  return ((uint64_t)k << 32) | (uint64_t)(0xFFFFFFFFu - id);
+  return (b & 0x80000000u) ? ~b : (b | 0x80000000u);
+}
+__device__ __forceinline__ uint64_t argmax_key(float v, uint32_t id) {
+  return ((uint64_t)argmax_order(v) << 32) | (uint64_t)(0xFFFFFFFFu - id);
 }
 __device__ __forceinline__ int32_t argmax_key_id(uint64_t key) {
   return key == 0 ? 0 : (int32_t)(0xFFFFFFFFu - (uint32_t)(key & 0xFFFFFFFFu));

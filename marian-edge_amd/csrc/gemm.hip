@@ -11,6 +11,7 @@
 // ReLU (tensor.rs:114-116), optional raw i32 store.
 #include "device_common.h"
 #include "kernels.h"
+#include <type_traits>
 #include <hip/hip_ext.h>
 
 namespace mh {
@@ -309,6 +310,12 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_skinny(GemmArgs g, Epilogue e)
 // reduction of accumulators is needed.  The activation rows are staged once
 // per workgroup in LDS.  Each row's best (logit, id) key over the workgroup's
 // columns is written as one partial; the step finalizer reduces the partials.
+//
+// Above 64 rows the epilogue bounds it: 64 x 128 outputs per workgroup.  With
+// a division and a 64-bit key per output, all keys parked in LDS (67 KB, two
+// workgroups per CU), 256 x 32000 (K = 512) took 29.0 us and 512 x 32000 49.9
+// with the reduction; with recip_exact, 32-bit key halves reduced by lane moves
+// and 36 KB (four per CU), 22.0 and 33.8 (64 rows: 13.6 -> 12.5).
 // ---------------------------------------------------------------------------
 constexpr int kVocabCols = 128;                   // columns per workgroup
 // Waves per workgroup: 8 of one column tile when the kernel builds the rows'
@@ -327,16 +334,15 @@ constexpr int kVocabLds = kVocabMaxK + 16;        // padded LDS row (bytes)
 // matrix cores read.
 // FAST (with LNP): the LayerNorm sums in the fast-reduction tree order.
 template <bool FULL, bool LNP, bool FAST = false>
-__global__ __launch_bounds__(64 * kVocabWaves<LNP>) void k_vocab_argmax(GemmArgs g, Epilogue e) {
+__global__ __launch_bounds__(64 * kVocabWaves<LNP>, 4) void k_vocab_argmax(GemmArgs g, Epilogue e) {
   touch_kernargs<sizeof(GemmArgs) + sizeof(Epilogue)>();
   constexpr int kVocabThreads = 64 * kVocabWaves<LNP>;
   constexpr int kVocabCT = kVocabCols / (16 * kVocabWaves<LNP>);  // column tiles per wave
-  constexpr int KEYS = kVocabWaves<LNP> * 16;  // per row: one key per (wave, lane column)
   static_assert(kVocabCT * 16 * kVocabWaves<LNP> == kVocabCols, "whole tiles per wave");
   static_assert(!LNP || (kVocabLnMaxRows <= kVocabWaves<LNP> && kVocabLnMaxRows <= 4), "a wave per prologue row");
   constexpr int PER = kVocabMaxK / 64;  // prologue rows: lane l holds elements l + 64j
   __shared__ __attribute__((aligned(16))) int8_t sA[kSkinnyRows * kVocabLds];
-  __shared__ uint64_t sK[kSkinnyRows * (KEYS + 1)];
+  __shared__ uint64_t sK[kVocabWaves<LNP> * kSkinnyRows];  // each wave's best key of a row
   __shared__ float sAm[kSkinnyRows];
   __shared__ __attribute__((aligned(16))) float sZ[LNP ? 4 * kLnRow<PER> : 4];
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
@@ -390,7 +396,7 @@ __global__ __launch_bounds__(64 * kVocabWaves<LNP>) void k_vocab_argmax(GemmArgs
   // requested at once.
   // The first chunk is requested for the rows below the host bound g.M (all
   // allocated) before the device row count arrives.
-  // Above 64 rows each 64-row group is a row of workgroups (blockIdx.y), so
+  // Each 64-row group is a row of workgroups (blockIdx.y), so
   // the groups run side by side; every group reads the weights again (from
   // the caches: the vocabulary is 16 MB).
   constexpr int kStage = kSkinnyRows * (kVocabMaxK / 16) / kVocabThreads;
@@ -431,121 +437,109 @@ __global__ __launch_bounds__(64 * kVocabWaves<LNP>) void k_vocab_argmax(GemmArgs
     }
   }
 
-  for (int m0 = r0; m0 < M; m0 += kSkinnyRows) {
-    const int rows = min(kSkinnyRows, M - m0);
-    if constexpr (!LNP) {
+  const int rows = M - r0;
+  if (rows <= 0) return;
+  if constexpr (!LNP) {
 #pragma unroll
-      for (int j = 0; j < kStage; ++j) {
-        const int c = tid + kVocabThreads * j;
-        *(v4i*)(sA + (c >> 5) * kVocabLds + (c & 31) * 16) = st[j];
-      }
-      if (tid < kSkinnyRows) sAm[tid] = sa;
-      // The next chunk's rows are requested now, from clamped (allocated)
-      // rows with the pieces past the chunk masked, so they arrive while this
-      // chunk is multiplied instead of after it.
-      const int m1 = m0 + kSkinnyRows, rows1 = M - m1;
-#pragma unroll
-      for (int j = 0; j < kStage; ++j) {
-        const int c = tid + kVocabThreads * j, row = c >> 5, cc = c & 31;
-        st[j] = keep_or_zero(*(const v4i*)(g.A + (int64_t)min(m1 + row, M - 1) * g.lda + min(cc, cpr - 1) * 16),
-                             row < rows1 && cc < cpr);
-      }
-      sa = g.a[min(m1 + tid, M - 1)];  // read only for rows of the chunk
+    for (int j = 0; j < kStage; ++j) {
+      const int c = tid + kVocabThreads * j;
+      *(v4i*)(sA + (c >> 5) * kVocabLds + (c & 31) * 16) = st[j];
     }
-    __syncthreads();
-    const int mt_n = (rows + 15) >> 4;
-    v4i acc[4][kVocabCT];
+    if (tid < kSkinnyRows) sAm[tid] = sa;
+  }
+  __syncthreads();
+  const int mt_n = (rows + 15) >> 4;
+  v4i acc[4][kVocabCT];
 #pragma unroll
-    for (int mt = 0; mt < 4; ++mt)
+  for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
-      for (int ct = 0; ct < kVocabCT; ++ct) acc[mt][ct] = zero4();
-    if (FULL && mt_n == 1) {
-      // One row tile (the common decode case): every k-step's A fragment is
-      // read at once, then the matrix cores run four independent chains
-      // (two column tiles x even / odd k-steps; exact integer sums).
-      constexpr int S = kVocabMaxK / 64;
-      v4i a1[S];
+    for (int ct = 0; ct < kVocabCT; ++ct) acc[mt][ct] = zero4();
+  if (FULL && mt_n == 1) {
+    // One row tile (the common decode case): every k-step's A fragment is
+    // read at once, then the matrix cores run four independent chains
+    // (two column tiles x even / odd k-steps; exact integer sums).
+    constexpr int S = kVocabMaxK / 64;
+    v4i a1[S];
 #pragma unroll
-      for (int s = 0; s < S; ++s) a1[s] = *(const v4i*)(sA + (lane & 15) * kVocabLds + kq + s * 64);
-      v4i acc2[kVocabCT];
+    for (int s = 0; s < S; ++s) a1[s] = *(const v4i*)(sA + (lane & 15) * kVocabLds + kq + s * 64);
+    v4i acc2[kVocabCT];
 #pragma unroll
-      for (int ct = 0; ct < kVocabCT; ++ct) acc2[ct] = zero4();
+    for (int ct = 0; ct < kVocabCT; ++ct) acc2[ct] = zero4();
 #pragma unroll
-      for (int s = 0; s < S; s += 2)
+    for (int s = 0; s < S; s += 2)
 #pragma unroll
-        for (int ct = 0; ct < kVocabCT; ++ct) {
-          acc[0][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1[s], bf[ct][s], acc[0][ct], 0, 0, 0);
-          acc2[ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1[s + 1], bf[ct][s + 1], acc2[ct], 0, 0, 0);
-        }
+      for (int ct = 0; ct < kVocabCT; ++ct) {
+        acc[0][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1[s], bf[ct][s], acc[0][ct], 0, 0, 0);
+        acc2[ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a1[s + 1], bf[ct][s + 1], acc2[ct], 0, 0, 0);
+      }
 #pragma unroll
-      for (int ct = 0; ct < kVocabCT; ++ct) acc[0][ct] += acc2[ct];
-    } else {
-      // All live row tiles advance together over K: up to 4 x kVocabCT
-      // independent accumulation chains keep the matrix core busy.
+    for (int ct = 0; ct < kVocabCT; ++ct) acc[0][ct] += acc2[ct];
+  } else {
+    // All live row tiles advance together over K: up to 4 x kVocabCT
+    // independent accumulation chains keep the matrix core busy.
 #pragma unroll
-      for (int s = 0; s < kVocabMaxK / 64; ++s) {
-        if (FULL || s < ksteps) {
+    for (int s = 0; s < kVocabMaxK / 64; ++s) {
+      if (FULL || s < ksteps) {
 #pragma unroll
-          for (int mt = 0; mt < 4; ++mt) {
-            if (mt < mt_n) {
-              const v4i af = *(const v4i*)(sA + (mt * 16 + (lane & 15)) * kVocabLds + kq + s * 64);
+        for (int mt = 0; mt < 4; ++mt) {
+          if (mt < mt_n) {
+            const v4i af = *(const v4i*)(sA + (mt * 16 + (lane & 15)) * kVocabLds + kq + s * 64);
 #pragma unroll
-              for (int ct = 0; ct < kVocabCT; ++ct)
-                acc[mt][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, bf[ct][s], acc[mt][ct], 0, 0, 0);
-            }
+            for (int ct = 0; ct < kVocabCT; ++ct)
+              acc[mt][ct] = __builtin_amdgcn_mfma_i32_16x16x64_i8(af, bf[ct][s], acc[mt][ct], 0, 0, 0);
           }
         }
       }
     }
-    // Lane holds rows 4*(lane/16)+r of each tile and column lane%16 of each of
-    // its column tiles: dequantize in registers, keep the best of its columns
-    // per row, and park it in LDS.
+  }
+  // Lane holds rows 4*(lane/16)+r of each tile and column lane%16 of each of
+  // its column tiles.  Each output is dequantized (recip_exact where every
+  // factor's exponent allows it, the IEEE division else) and turned into the
+  // upper half of its argmax key; per row the largest over the wave's columns,
+  // and the lowest id among those equal to it, are found with lane moves
+  // within the 16 lanes that share the row.
+  bool ok = lane >= rows || recip_factor(sAm[lane]);
+#pragma unroll
+  for (int ct = 0; ct < kVocabCT; ++ct) ok = ok && recip_factor(wm[ct]);
+  const bool fast = __all(ok);
+  auto rows_best = [&](auto quick) {
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
       if (mt < mt_n) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           const int lr = mt * 16 + (lane >> 4) * 4 + r;
-          uint64_t key = 0;
-          if (lr < rows) {
-            const int m = m0 + lr;
-            const float am = sAm[lr];
+          const float am = sAm[lr];
+          uint32_t key = 0, id = 0;
 #pragma unroll
-            for (int ct = 0; ct < kVocabCT; ++ct) {
-              const float y = dequant(acc[mt][ct][r], am, wm[ct], bi[ct]);
-              if (e.logits && ncol[ct] < g.N)
-                e.logits[(int64_t)m * e.ldl + ncol[ct]] = live[ct] ? y : -INFINITY;
-              if (live[ct]) {
-                const uint64_t k = argmax_key(y, (uint32_t)ncol[ct]);
-                key = k > key ? k : key;
-              }
+          for (int ct = 0; ct < kVocabCT; ++ct) {
+            const float w = am * wm[ct];
+            const float y = dequant_apply(acc[mt][ct][r], quick ? recip_exact(w) : 1.0f / w, bi[ct]);
+            if (e.logits && ncol[ct] < g.N && lr < rows)
+              e.logits[(int64_t)(r0 + lr) * e.ldl + ncol[ct]] = live[ct] ? y : -INFINITY;
+            const uint32_t k = live[ct] ? argmax_order(y) : 0u;
+            if (ct == 0 || k > key) {  // ids ascend: the first of equals stays
+              key = k;
+              id = (uint32_t)ncol[ct];
             }
           }
-          sK[lr * (KEYS + 1) + wave * 16 + (lane & 15)] = key;
+          const uint32_t best = row16_max(key);
+          const uint32_t inv = row16_max(key == best ? ~id : 0u);  // the lowest id has the largest complement
+          if ((lane & 15) == 0) sK[wave * kSkinnyRows + lr] = best ? ((uint64_t)best << 32) | inv : 0u;
         }
       }
     }
-    __syncthreads();
-    // P threads per row reduce its KEYS parked keys.
-    {
-      constexpr int P = kVocabThreads / kSkinnyRows;
-      static_assert(P == 4 || P == 8, "4 or 8 threads per row");
-      const int row = tid / P, part = tid % P;
-      uint64_t best = 0;
-      if (row < rows) {
+  };
+  if (fast)
+    rows_best(std::true_type());
+  else
+    rows_best(std::false_type());
+  __syncthreads();
+  if (tid < rows) {
+    uint64_t best = sK[tid];
 #pragma unroll
-        for (int j = 0; j < KEYS / P; ++j) {
-          const uint64_t k = sK[row * (KEYS + 1) + part * (KEYS / P) + j];
-          best = k > best ? k : best;
-        }
-      }
-      best = umax64(best, xor_lane_u64<1>(best));
-      best = umax64(best, xor_lane_u64<2>(best));
-      if constexpr (P == 8) best = umax64(best, xor_lane_u64<4>(best));
-      if (row < rows && part == 0)
-        e.partials[(int64_t)(m0 + row) * e.partial_ld + blockIdx.x] = best;
-    }
-    __syncthreads();
+    for (int w = 1; w < kVocabWaves<LNP>; ++w) best = umax64(best, sK[w * kSkinnyRows + tid]);
+    e.partials[(int64_t)(r0 + tid) * e.partial_ld + blockIdx.x] = best;
   }
 }
 

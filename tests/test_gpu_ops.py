@@ -605,6 +605,35 @@ def test_vocab_argmax_nonfinite_logits_follow_strict_scan(pkg, dev):
     assert run(b) == [50, 50]
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,K,V", [(1, 64, 40), (17, 512, 130), (64, 384, 4097), (70, 512, 300), (200, 256, 1000)])
+@pytest.mark.parametrize("scale", [0, 70, -90])
+def test_vocab_argmax_ties_and_factors(pkg, dev, M, K, V, scale):
+    """Logits and tokens against IEEE float32 arithmetic: multipliers within the
+    short reciprocal's exponents and, scaled by 2^scale in one column, outside
+    them; duplicate columns, so equal logits must keep the lowest id across
+    lanes, column tiles, waves and workgroups."""
+    print(f"vocab_argmax M={M} K={K} V={V} scale={scale}", flush=True)
+    rng = np.random.default_rng(7)
+    emb = rng.integers(-127, 128, (V, K)).astype(np.int8)
+    emb[V // 2:] = emb[: V - V // 2]  # every column at least twice
+    mult = np.full(V, 37.5, np.float32)
+    bias = np.full(V, 0.25, np.float32)
+    mult[V - 1] *= np.float32(2.0) ** scale
+    xq = rng.integers(-127, 128, (M, K)).astype(np.int8)
+    xa = rng.uniform(1.0, 300.0, M).astype(np.float32)
+    acc = (xq.astype(np.int32) @ emb.astype(np.int32).T).astype(np.float32)
+    ref = acc * (np.float32(1) / (xa[:, None] * mult[None, :])) + bias
+    assert ref.dtype == np.float32
+    ids = np.arange(V)
+    ref[:, (ids == 1) | ((ids >= 7) & (ids <= 38))] = -np.inf
+    tok, logits = dev.DeviceArray.zeros(M, np.int32), dev.DeviceArray.zeros((M, V), np.float32)
+    dev.vocab_argmax(*(dev.DeviceArray.from_host(t) for t in (xq, xa, emb, mult, bias)), tok, logits=logits)
+    dev.synchronize()
+    assert np.array_equal(logits.host().view(np.uint32), ref.view(np.uint32))
+    assert np.array_equal(tok.host(), np.argmax(ref, axis=1).astype(np.int32))
+
+
 # ---- static activation multiplier (the reference's Q8 models) ---------------------
 @pytest.mark.parametrize("K,N", [(512, 1536), (2048, 512), (512, 32000)])
 @pytest.mark.parametrize("M", [1, 8, 64, 256])
