@@ -540,11 +540,14 @@ __global__ __launch_bounds__(256) void k_argmax_reduce(const uint64_t* partials,
                                                        int rows, int32_t* token) {
   const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= rows) return;
-  uint64_t best = 0;
-  for (int p = lane; p < nparts; p += 64) {
-    const uint64_t k = partials[(int64_t)row * nparts + p];
-    best = k > best ? k : best;
-  }
+  // The first 256 partials (32768 columns) are requested together: one memory
+  // round trip instead of one per 64 (the 64 x 32000 argmax call 12.44 -> 11.73 us).
+  const uint64_t* pr = partials + (int64_t)row * nparts;
+  uint64_t v[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) v[k] = pr[min(lane + 64 * k, nparts - 1)];  // repeats leave the maximum
+  uint64_t best = umax64(umax64(v[0], v[1]), umax64(v[2], v[3]));
+  for (int p = lane + 256; p < nparts; p += 64) best = umax64(best, pr[p]);
   best = wave_max_u64(best);
   if (lane == 0) token[row] = argmax_key_id(best);
 }

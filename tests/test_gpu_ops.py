@@ -606,7 +606,8 @@ def test_vocab_argmax_nonfinite_logits_follow_strict_scan(pkg, dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,K,V", [(1, 64, 40), (17, 512, 130), (64, 384, 4097), (70, 512, 300), (200, 256, 1000)])
+@pytest.mark.parametrize("M,K,V", [(1, 64, 40), (17, 512, 130), (64, 384, 4097), (70, 512, 300), (200, 256, 1000),
+                                   (3, 64, 33000)])
 @pytest.mark.parametrize("scale", [0, 70, -90])
 def test_vocab_argmax_ties_and_factors(pkg, dev, M, K, V, scale):
     """Logits and tokens against IEEE float32 arithmetic: multipliers within the
