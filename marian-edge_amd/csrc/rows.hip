@@ -164,6 +164,120 @@ __global__ __launch_bounds__(256) void k_residual_ln(const float* y, const float
   ln_row_wave<PER, FAST>(z, sZ[wave], gv, bv, row, lane, out, q, a, err, qmult);
 }
 
+// The same for many rows (no device row count, no static multiplier): R rows
+// per wave, each lane holding V consecutive elements at a time, and the rows'
+// sequential folds side by side, lane = row.  Widths without the speculative
+// folds otherwise take a whole wave for one row's chains; with them, the
+// candidates (64 lanes reading every term) cost more than the shorter chains
+// save once enough rows are in flight, except at 512.  Whole calls on changing
+// inputs, one row per wave -> here, us: 2700 rows of 640 12.5 -> 10.6, of 1024
+// 18.9 -> 15.6; 7405 rows of 256 8.65 -> 8.18, of 384 11.2 -> 10.8, of 512 13.1 ->
+// 13.4; 16384 rows of 256 14.6 -> 12.1, of 384 19.0 -> 15.4, of 512 25.4 -> 25.2.
+// Fewer rows leave the chip idle and the longer chains show (4500 rows of 384
+// 8.25 -> 9.80; 1459 of 1024 11.9 -> 15.2).
+template <int PER>
+constexpr int kLnManyRows = PER == 8 ? INT32_MAX : (kLnSpec<PER> ? 7168 : 2560);
+template <int PER>
+constexpr int kLnR = PER <= 8 ? 4 : 2;
+template <int V>
+using LnPiece = float __attribute__((ext_vector_type(V), aligned(4)));  // rows are aligned as floats only
+typedef uint32_t ln_u32 __attribute__((aligned(1)));
+typedef uint16_t ln_u16 __attribute__((aligned(1)));
+
+template <int PER, int R>
+__global__ __launch_bounds__(256) void k_residual_ln_rows(const float* y, const float* r, const float* gamma,
+                                                          const float* beta, int rows, float* out, int8_t* q,
+                                                          float* a, int* err) {
+  constexpr int D = PER * 64, S = D + 4;
+  constexpr int V = PER % 4 == 0 ? 4 : (PER % 2 == 0 ? 2 : 1), NV = PER / V;
+  __shared__ __attribute__((aligned(16))) float sZ[4][R * S];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int row0 = (blockIdx.x * 4 + wave) * R;
+  if (row0 >= rows) return;  // uniform per wave; the waves share no barrier
+  // Element V k + v of a lane's row is column 64 V k + V lane + v.
+  auto load = [&](const float* p, float (&x)[PER]) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      const LnPiece<V> w = *(const LnPiece<V>*)(p + V * lane + 64 * V * k);
+#pragma unroll
+      for (int v = 0; v < V; ++v) x[V * k + v] = w[v];
+    }
+  };
+  float z[R][PER], gv[PER], bv[PER];
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const int64_t ro = (int64_t)min(row0 + i, rows - 1) * D;
+    float t[PER];
+    load(y + ro, z[i]);
+    load(r + ro, t);
+#pragma unroll
+    for (int j = 0; j < PER; ++j) z[i][j] = z[i][j] + t[j];
+  }
+  load(gamma, gv);
+  load(beta, bv);
+  float* zr = sZ[wave];
+  auto fold = [&](float (&v)[R][PER], bool centred, const float (&mean)[R]) {
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const float c = v[i][j] - mean[i];
+        zr[i * S + V * lane + 64 * V * (j / V) + j % V] = centred ? c * c : v[i][j];
+      }
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the rows are in LDS
+    __builtin_amdgcn_wave_barrier();
+    float s = 0.0f;
+    if (lane < R) s = seq_fold_lds<D / 4>((const float4*)(zr + lane * S), -0.0f);
+    __builtin_amdgcn_wave_barrier();
+    return s;
+  };
+  float mean[R] = {};
+  float s = fold(z, false, mean) / (float)D;
+#pragma unroll
+  for (int i = 0; i < R; ++i) mean[i] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), i));
+  s = 1.0f / sqrtf(fold(z, true, mean) / (float)D + kLayerNormEpsilon);
+  bool bad = false;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const float inv = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s), i));
+    const int row = row0 + i;
+    if (row >= rows) break;
+    float o[PER], m = 0.0f;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+      o[j] = ((z[i][j] - mean[i]) * inv) * gv[j] + bv[j];
+      bad |= !isfinite(o[j]);
+      m = fmaxf(m, fabsf(o[j]));
+    }
+    const int64_t ro = (int64_t)row * D + V * lane;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      LnPiece<V> w;
+#pragma unroll
+      for (int v = 0; v < V; ++v) w[v] = o[V * k + v];
+      *(LnPiece<V>*)(out + ro + 64 * V * k) = w;
+    }
+    if (q) {
+      const float sc = row_multiplier(wave_max(m));
+#pragma unroll
+      for (int k = 0; k < NV; ++k) {
+        uint32_t w = 0;
+#pragma unroll
+        for (int v = 0; v < V; ++v) w |= (uint32_t)(quantize_one(o[V * k + v], sc) & 0xFF) << (8 * v);
+        int8_t* p = q + ro + 64 * V * k;
+        if constexpr (V == 4)
+          *(ln_u32*)p = w;
+        else if constexpr (V == 2)
+          *(ln_u16*)p = (uint16_t)w;
+        else
+          *p = (int8_t)w;
+      }
+      if (lane == 0) a[row] = sc;
+    }
+  }
+  if (__any(bad) && lane == 0 && err) *err = 1;
+}
+
 // SSRU state update + LayerNorm (ssru_update_layer_norm_into, tensor.rs:184-218,
 // the reference's SSRU decoder, q8_engine.rs:394-408).  Per element: gate =
 // 1 / (1 + exp(-f)) with the C library's expf, s' = gate * s + (1 - gate) * c
@@ -602,12 +716,21 @@ hipError_t launch_quantize_rows(const float* x, int64_t ldx, int rows, const int
     default: return hipErrorInvalidValue;   \
   }
 
+template <int PER>
+static void launch_ln_rows(const float* y, const float* r, const float* g, const float* b, int rows, float* out,
+                           int8_t* q, float* a, int* err, hipStream_t s) {
+  if constexpr (PER != 8) {  // rows of 512 keep one wave each
+    constexpr int R = kLnR<PER>;
+    hipLaunchKernelGGL((k_residual_ln_rows<PER, R>), dim3((rows + 4 * R - 1) / (4 * R)), dim3(256), 0, s, y, r, g, b,
+                       rows, out, q, a, err);
+  }
+}
 hipError_t launch_residual_ln(const float* y, const float* r, const float* g, const float* b,
                               int rows, const int* rows_dev, int d, float* out, int8_t* q,
                               float* a, int* err, hipStream_t s, float qmult, bool fast) {
   if (rows <= 0) return hipSuccess;
   if (d % 64) return hipErrorInvalidValue;
-  // One wave per row, four rows per workgroup: widths of 256, 384 and 512
+  // Many rows: several per wave.  Else one wave per row, four rows per workgroup: widths of 256, 384 and 512
   // fold with the one-wave speculative folds, others sequentially; with
   // `fast` (the decoder's widths) the sums take the tree order.
   const dim3 grid((rows + 3) / 4), block(256);
@@ -616,11 +739,16 @@ hipError_t launch_residual_ln(const float* y, const float* r, const float* g, co
 #define MH_LNF(P)                                                                                            \
   hipLaunchKernelGGL((k_residual_ln<P, true>), grid, block, 0, s, y, r, g, b, rows, rows_dev, out, q, a, err, \
                      qmult)
-  if (fast) {
+  const int many = d == 512 ? kLnManyRows<8> : (d == 256 || d == 384 ? kLnManyRows<4> : kLnManyRows<1>);
+  if (!fast && !rows_dev && !(qmult > 0.0f) && rows >= many) {
+#define MH_LNR(P) launch_ln_rows<P>(y, r, g, b, rows, out, q, a, err, s)
+    MH_PER_DISPATCH_16(d / 64, MH_LNR)
+  } else if (fast) {
     MH_PER_DISPATCH(d / 64, MH_LNF)
   } else {
     MH_PER_DISPATCH_16(d / 64, MH_LN)
   }
+#undef MH_LNR
 #undef MH_LNF
 #undef MH_LN
   return hipGetLastError();

@@ -275,6 +275,40 @@ def test_residual_layer_norm_matches_oracle(pkg, orc, dev):
         assert np.array_equal(q.host(), q_ref) and np.array_equal(a.host(), a_ref)
 
 
+@pytest.mark.parametrize("d,rows", [(64, 2560), (192, 2561), (256, 7168), (256, 7171), (384, 7169), (512, 7405),
+                                    (640, 2563), (960, 2561), (1024, 2562)])
+def test_residual_layer_norm_many_rows(pkg, orc, dev, d, rows):
+    """Several rows per wave: every width's lane layout, a last wave with fewer
+    rows, rows that start at any float, and non-finite rows."""
+    print(f"residual_layer_norm {rows} x {d}", flush=True)
+    rng = np.random.default_rng(29)
+    y = rng.standard_normal((rows, d)).astype(np.float32)
+    r = (rng.standard_normal((rows, d)) * 3).astype(np.float32)
+    y[0], r[0] = 0.0, -0.0
+    y[rows - 1, d - 1], y[rows - 2, 0] = np.inf, np.nan
+    g = (1 + 0.1 * rng.standard_normal(d)).astype(np.float32)
+    b = (0.1 * rng.standard_normal(d)).astype(np.float32)
+    ref = orc.residual_layer_norm(y, r, g, b)
+    q_ref, a_ref = orc.quantize_rows(ref[: rows - 2])
+
+    class Shifted:  # the buffer one element past its start
+        def __init__(self, host):
+            self.whole = dev.DeviceArray.from_host(np.concatenate([host.reshape(-1)[:1], host.reshape(-1)]))
+            self.shape, self.ptr = host.shape, self.whole.ptr + host.itemsize
+
+    out, q = Shifted(np.zeros_like(y)), Shifted(np.zeros(y.shape, np.int8))
+    a = dev.DeviceArray.zeros(rows, np.float32)
+    err = dev.DeviceArray.zeros(1, np.int32)
+    dev.residual_layer_norm(Shifted(y), Shifted(r), Shifted(g), Shifted(b), out, q, a, err=err)
+    dev.synchronize()
+    got = out.whole.host()[1:].reshape(rows, d)
+    fin = slice(0, rows - 2)
+    assert np.array_equal(got[fin].view(np.uint32), ref[fin].view(np.uint32))
+    assert np.array_equal(np.isnan(got), np.isnan(ref)) and err.host()[0] == 1
+    assert np.array_equal(q.whole.host()[1:].reshape(rows, d)[fin], q_ref)
+    assert np.array_equal(a.host()[fin], a_ref)
+
+
 def _ln_edge_rows(rng, d=512):
     """Rows whose sequential sums stress the speculative folds (chunks of 64
     or 128):
