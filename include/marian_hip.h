@@ -414,7 +414,8 @@ int marian_hip_quantize_rows(const float* x, int64_t rows, int64_t cols, int8_t*
 
 /* y = (x quantized per row) @ W^T dequantized + bias (+ReLU).
  * x fp32 [M,K] (NULL when xq/xa are given pre-quantized), W int8 [N,K],
- * out_i32 [M,N] optional (exact accumulators), out_f32 [M,N] optional.
+ * out_i32 [M,N] optional (exact accumulators), out_f32 [M,N] optional; either
+ * may share memory with x (e.g. out_f32 = x for K = N).
  * K must be a multiple of 64. */
 int marian_hip_q8_linear(const float* x, const int8_t* xq, const float* xa, int64_t M,
                          int64_t K, const int8_t* w, const float* w_mult, const float* bias,

@@ -115,9 +115,15 @@ int vocab_argmax_into(const int8_t* xq, const float* xa, int64_t M, int64_t K, c
   return op_status(launch_argmax_reduce(part, nparts, (int)M, token, s), "vocab_argmax reduce");
 }
 
+bool overlap(const void* a, size_t na, const void* b, size_t nb) {
+  return a && b && (uintptr_t)a < (uintptr_t)b + nb && (uintptr_t)b < (uintptr_t)a + na;
+}
+
 // A Q8 layer from fp32 rows x (each row's own multiplier, or the static `act`
 // when positive) or, without x, from quantized rows: one launch where
 // linear_f32_fused says so, else the row quantization into scratch first.
+// An output that shares memory with x always takes the latter: in one launch
+// a workgroup would store its columns over rows that others still quantize.
 int linear_op(const float* x, float act, const int8_t* xq, const float* xa, int64_t M, int64_t K, const int8_t* w,
               const float* w_mult, const float* bias, int64_t N, int relu, int32_t* out_i32, float* out_f32, int* err,
               hipStream_t s, const char* what) {
@@ -140,7 +146,9 @@ int linear_op(const float* x, float act, const int8_t* xq, const float* xa, int6
     g.ldaf = K;
     g.act = act;
     g.err = err;
-    if (linear_f32_fused(g, e)) return op_status(launch_linear_f32(g, e, s), what);
+    const size_t in = (size_t)M * K * 4, res = (size_t)M * N * 4;
+    const bool in_place = overlap(x, in, out_f32, res) || overlap(x, in, out_i32, res);
+    if (!in_place && linear_f32_fused(g, e)) return op_status(launch_linear_f32(g, e, s), what);
     g.Af = nullptr;
     g.err = nullptr;
     int8_t* q = (int8_t*)op_scratch(0, (size_t)M * K, s);

@@ -169,6 +169,56 @@ def test_q8_linear_from_fp32_rows(dev, M, K, N, act):
                 assert np.array_equal(gi.host(), wi.host())
 
 
+class _Part:
+    """Elements [first, ...) of a device buffer as an array of its own."""
+
+    def __init__(self, whole, first, shape, dtype):
+        self.whole, self.shape, self.dtype = whole, shape, np.dtype(dtype)
+        self.ptr = whole.ptr + 4 * first
+
+    def host(self):
+        n = int(np.prod(self.shape))
+        first = (self.ptr - self.whole.ptr) // 4
+        return self.whole.host().reshape(-1).view(self.dtype)[first:first + n].reshape(self.shape)
+
+
+@pytest.mark.parametrize("act", [0.0, 31.75])
+@pytest.mark.parametrize("M,K,N", [(61, 384, 384), (64, 512, 512), (1459, 512, 512), (1459, 512, 1536), (50, 2048, 512)])
+def test_q8_linear_outputs_over_the_input(dev, M, K, N, act):
+    """Outputs that share memory with the fp32 rows they are computed from (the
+    same buffer, the rows' second half, the int32 copy over the rows) equal the
+    out-of-place call's, bit for bit, on every call of several."""
+    print(f"q8_linear in place M={M} K={K} N={N} act={act}", flush=True)
+    rng = np.random.default_rng(M + K)
+    D = dev.DeviceArray
+    x = rng.standard_normal((M, K)).astype(np.float32)
+    dw = D.from_host(rng.integers(-127, 128, size=(N, K)).astype(np.int8))
+    dm = D.from_host(rng.uniform(50, 100, size=N).astype(np.float32))
+    db = D.from_host(rng.standard_normal(N).astype(np.float32))
+
+    def call(dx, i32, f32):
+        if act:
+            dev.q8_linear_static(dx, act, dw, dm, db, i32, f32)
+        else:
+            dev.q8_linear(dx, dw, dm, db, i32, f32)
+        dev.synchronize()
+
+    wi, wf = D.zeros((M, N), np.int32), D.zeros((M, N), np.float32)
+    call(D.from_host(x), wi, wf)
+    size = M * (K + N)
+    for first_in, first_out in ((0, 0), (0, M * K // 2), (M * N // 2, 0)):
+        for ints in (False, True):
+            for _ in range(3):
+                whole = np.zeros(size, np.float32)
+                whole[first_in:first_in + M * K] = x.reshape(-1)
+                buf = D.from_host(whole)
+                dx = _Part(buf, first_in, (M, K), np.float32)
+                out = _Part(buf, first_out, (M, N), np.int32 if ints else np.float32)
+                call(dx, *((out, None) if ints else (None, out)))
+                want = wi if ints else wf
+                assert np.array_equal(out.host().view(np.uint32), want.host().view(np.uint32)), (first_in, first_out, ints)
+
+
 def test_q8_linear_on_two_streams_at_once(pkg, orc, dev):
     """The op-level entry points keep their intermediate buffers (here the
     quantized activations of an fp32 input) per (device, stream): two streams
