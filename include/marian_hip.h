@@ -452,7 +452,7 @@ int marian_hip_residual_layer_norm(const float* x, const float* r, const float* 
  * and attends over key rows [cu_k[s], cu_k[s+1]); max_keys bounds every range
  * (at most 4096); heads <= 16 of width head_dim (64, or 48 as in the
  * reference's 384-wide model; head h is columns [h*head_dim, (h+1)*head_dim)).
- * Row strides in elements.  in_bf16 != 0 reads q/k/v as bfloat16 (converted
+ * Row strides in elements, any multiples of 8.  in_bf16 != 0 reads q/k/v as bfloat16 (converted
  * exactly to fp32); out is fp32 [rows, heads*head_dim].
  * n_seqs > 0 declares packed self-attention: the query rows are the key rows
  * (row i lies in [cu_k[s], cu_k[s+1]) for s = seq_of_row[i]), cu_k has

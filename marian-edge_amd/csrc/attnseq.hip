@@ -64,7 +64,8 @@ __constant__ uint64_t kSeqExp2Tab[32] = {MH_EXP2_TABLE_32};
 // n rows of ld elements from p on, of which the last holds `width` elements, as
 // a raw buffer resource: a load at or past its end returns zeros (the hardware
 // range check on the VGPR offset), so one lane offset serves every row block
-// and rows past the last need no mask.  n ld sizeof(T) < 2^32.
+// and rows past the last need no mask.  It needs width <= ld and every offset
+// below 2^32 bytes (seq_buffer_rows).
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 constexpr int kRawBufferWord3 = 0x00020000;  // gfx9 raw buffer: 32-bit data format, no swizzle
@@ -89,6 +90,13 @@ __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t r, uint32_t off, f
 __device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t r, uint32_t off, uint16_t) {
   return bf16_to_f32(__builtin_amdgcn_raw_buffer_load_b16(r, off, 0, 0));
 }
+// The same through a pointer with its element's alignment (general strides).
+typedef u32x4 u32x4u __attribute__((aligned(4)));
+typedef u32x2 u32x2u __attribute__((aligned(2)));
+__device__ __forceinline__ u32x4 load4(const float* p) { return *(const u32x4u*)p; }
+__device__ __forceinline__ u32x2 load4(const uint16_t* p) { return *(const u32x2u*)p; }
+__device__ __forceinline__ float load1(const float* p) { return *p; }
+__device__ __forceinline__ float load1(const uint16_t* p) { return bf16_to_f32(*p); }
 
 // A wave's tile of QW queries x 64 keys (or dimensions): register 4b + r of
 // lane l holds column l % QW and row 4 (64 / QW) b + 4 (l / QW) + r.
@@ -257,7 +265,9 @@ __device__ __forceinline__ bool find_unit(const uint32_t* cu, int n, int heads, 
 
 // CH: 64-key chunks whose scores the registers hold (4: 256 keys; 8: 512 keys).
 // QW: queries per wave.
-template <int CH, int QW, typename T, int DH>
+// GEN: rows by 64-bit addresses, for the strides and alignments that
+// seq_buffer_rows refuses (any stride, overlapping rows, odd bf16 addresses).
+template <int CH, int QW, typename T, int DH, bool GEN>
 __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) void k_attn_seq(AttnArgs a) {
   static_assert(DH == 64 || DH == 48, "head widths");
   constexpr int W = kSeqWaves, TQ = W * QW;  // queries per workgroup
@@ -324,6 +334,16 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
   }
   const int nh = min(hpw, a.heads - h0);
   auto request = [&](const T* src, int c) {
+    if constexpr (GEN) {
+#pragma unroll
+      for (int i = 0; i < NP; ++i) {
+        const int row = (tid >> 4) + 4 * W * i, hs = row / sp, key = 64 * c + row - hs * sp;
+        pre[i] = {};
+        if (key < Lc && hs < nh)
+          pre[i] = load4(src + (key0 + key) * a.ldkv + (h0 + hs) * DH + min((tid & 15) * 4, DH - 4));
+      }
+      return;
+    }
     const __amdgpu_buffer_rsrc_t r =
         rows_of(src + (key0 + 64 * c) * a.ldkv + (int64_t)h0 * DH, min(Lc - 64 * c, sp), a.ldkv, nh * DH);
 #pragma unroll
@@ -339,11 +359,19 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
   const bool live = nq > 0 && h < a.heads;  // uniform per wave
   request(kp, 0);
   if (live) {
-    const __amdgpu_buffer_rsrc_t r = rows_of(qp + (key0 + qw) * a.ldq + h * DH, nq, a.ldq, DH);
     float qv[QW];
+    if constexpr (GEN) {
 #pragma unroll
-    for (int i = 0; i < QW; ++i)
-      qv[i] = load1(r, ((uint32_t)i * (uint32_t)a.ldq + min(lane, DH - 1)) * (uint32_t)sizeof(T), T());
+      for (int i = 0; i < QW; ++i) {
+        qv[i] = 0.0f;
+        if (i < nq) qv[i] = load1(qp + (key0 + qw + i) * a.ldq + h * DH + min(lane, DH - 1));
+      }
+    } else {
+      const __amdgpu_buffer_rsrc_t r = rows_of(qp + (key0 + qw) * a.ldq + h * DH, nq, a.ldq, DH);
+#pragma unroll
+      for (int i = 0; i < QW; ++i)
+        qv[i] = load1(r, ((uint32_t)i * (uint32_t)a.ldq + min(lane, DH - 1)) * (uint32_t)sizeof(T), T());
+    }
 #pragma unroll
     for (int i = 0; i < QW; ++i) sP[i * kSeqRow + lane] = qv[i];
   }
@@ -458,19 +486,28 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
   }
 }
 
-template <int CH, int QW, typename T>
+template <int CH, int QW, typename T, bool GEN>
 void launch_dh(const AttnArgs& a, dim3 grid, hipStream_t s) {
   if (a.head_dim == 48)
-    hipLaunchKernelGGL((k_attn_seq<CH, QW, T, 48>), grid, dim3(64 * kSeqWaves), 0, s, a);
+    hipLaunchKernelGGL((k_attn_seq<CH, QW, T, 48, GEN>), grid, dim3(64 * kSeqWaves), 0, s, a);
   else
-    hipLaunchKernelGGL((k_attn_seq<CH, QW, T, 64>), grid, dim3(64 * kSeqWaves), 0, s, a);
+    hipLaunchKernelGGL((k_attn_seq<CH, QW, T, 64, GEN>), grid, dim3(64 * kSeqWaves), 0, s, a);
 }
-template <int CH, int QW>
+template <int CH, int QW, bool GEN = false>
 void launch_t(const AttnArgs& a, dim3 grid, hipStream_t s) {
   if (a.bf16)
-    launch_dh<CH, QW, uint16_t>(a, grid, s);
+    launch_dh<CH, QW, uint16_t, GEN>(a, grid, s);
   else
-    launch_dh<CH, QW, float>(a, grid, s);
+    launch_dh<CH, QW, float, GEN>(a, grid, s);
+}
+
+// Whether the rows fit the kernel's raw buffers: 64 key rows (16 query rows)
+// within 32-bit offsets, no row reaching into the next (a row past the range's
+// end has to lie past it in every head), 4-byte aligned four-element loads.
+bool seq_buffer_rows(const AttnArgs& a) {
+  const int64_t d = (int64_t)a.heads * a.head_dim, size = a.bf16 ? 2 : 4, top = int64_t(1) << 32;
+  return a.ldq >= d && a.ldkv >= d && a.ldkv < top / (64 * size) && a.ldq < top / (16 * size) &&
+         ((uintptr_t)a.k | (uintptr_t)a.v) % 4 == 0;
 }
 
 }  // namespace
@@ -479,13 +516,16 @@ hipError_t launch_attention_seq(const AttnArgs& a, hipStream_t s) {
   if (a.mode != ATT_SEQ || a.n_seqs <= 0 || a.max_keys <= 0 || a.max_keys > kSeqMaxKeys || !a.cu ||
       (int64_t)a.n_seqs * a.heads > 0x7fffffff || (int64_t)a.rows * a.heads > 0x7fffffff)
     return hipErrorInvalidValue;
-  const bool few = (int64_t)a.rows * a.heads <= (a.max_keys <= 256 ? kSeqFewRows256 : kSeqFewRows512);
+  const bool gen = !seq_buffer_rows(a);
+  const bool few = !gen && (int64_t)a.rows * a.heads <= (a.max_keys <= 256 ? kSeqFewRows256 : kSeqFewRows512);
   const int tq = kSeqWaves * (few ? 4 : 16);
   // Units: at most heads / 4 + 7 / 256 heads L of a sequence of L rows (equal at 65 rows).
   const int64_t units = (int64_t)a.n_seqs * ((a.heads + 3) / 4) + ((int64_t)a.rows * a.heads * 7 + 255) / 256;
   const dim3 grid = !few && a.n_seqs <= kSeqFindMax ? dim3((uint32_t)units)
                                                     : dim3(a.n_seqs * a.heads, (a.max_keys + tq - 1) / tq);
-  if (a.max_keys <= 256)
+  if (gen)
+    launch_t<8, 16, true>(a, grid, s);
+  else if (a.max_keys <= 256)
     few ? launch_t<4, 4>(a, grid, s) : launch_t<4, 16>(a, grid, s);
   else
     few ? launch_t<8, 4>(a, grid, s) : launch_t<8, 16>(a, grid, s);

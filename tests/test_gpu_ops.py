@@ -594,6 +594,67 @@ def test_packed_attention_units(pkg, orc, dev, heads, head_dim, bf16, lens):
     assert np.array_equal(np.where(nan, 0, got).view(np.uint32), np.where(nan, 0, ref).view(np.uint32))
 
 
+class _Rows:
+    """n rows of d elements, ld elements apart, the first at element `first` of a
+    buffer that holds `size` elements; the bytes between the rows are 0xFF (NaN)."""
+
+    def __init__(self, dev, rows, ld, size, first):
+        self.whole = dev.DeviceArray(size, rows.dtype)
+        self.whole.fill_bytes(0xFF)
+        self.shape = (rows.shape[0], ld)  # the row stride, as the calls take it
+        item = rows.dtype.itemsize
+        self.ptr = self.whole.ptr + first * item
+        for i, row in enumerate(np.ascontiguousarray(rows)):
+            at = first + i * ld
+            assert 0 <= at and at + rows.shape[1] <= size
+            dev._lib.check(self.whole._lib.marian_hip_memcpy_h2d(self.ptr + i * ld * item, row.ctypes.data,
+                                                                 row.nbytes), "h2d")
+
+
+@pytest.mark.parametrize("heads,head_dim,bf16,lens,ldq,ldkv,shift", [
+    # key rows whose 64-row chunk, query rows whose 4-row group spans more than 2^32 bytes
+    (2, 64, False, [70, 3], None, 33 << 19, 0), (2, 48, True, [70, 3], None, 33 << 20, 0),
+    (2, 64, False, [3, 5], 3 << 27, None, 0), (1, 64, True, [3, 5], 3 << 28, None, 0),
+    # the widest strides of the path that addresses them by 32 bits
+    (2, 64, False, [66], None, (1 << 24) - 8, 0), (2, 64, False, [3, 5], (1 << 26) - 8, None, 0),
+    # one row for every key or query, rows that overlap, rows that go backwards
+    (4, 64, False, [5, 20, 70], 0, 0, 0), (4, 48, True, [5, 20, 70], 0, 0, 0),
+    (4, 64, False, [16, 9, 33, 257], None, 8, 0), (3, 48, True, [16, 9, 33], None, 136, 0),
+    (4, 64, False, [16, 9, 33, 130], -256, -264, 0), (4, 64, True, [16, 9, 33, 130], -264, -256, 0),
+    # buffers that start at an odd element
+    (4, 64, True, [16, 9, 33, 130], None, None, 1), (4, 64, False, [16, 9, 33, 130], None, None, 1),
+    (2, 64, True, [1 + (11 * i) % 70 for i in range(1030)], None, None, 1),
+])
+def test_packed_attention_row_strides(pkg, orc, dev, heads, head_dim, bf16, lens, ldq, ldkv, shift):
+    """Any row stride that is a multiple of 8 elements and any element alignment:
+    bit-identical to the oracle on the rows that the strides name."""
+    print(f"packed attention heads={heads} head_dim={head_dim} bf16={bf16} ldq={ldq} ldkv={ldkv}", flush=True)
+    rng = np.random.default_rng(43)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    T, d = int(cu[-1]), heads * head_dim
+
+    def rows(ld):
+        ld = d if ld is None else ld
+        if abs(ld) >= d:
+            x = rng.standard_normal((T, d)).astype(np.float32)
+        else:  # overlapping rows of one array
+            flat = rng.standard_normal((T - 1) * ld + d).astype(np.float32)
+            x = np.lib.stride_tricks.as_strided(flat, (T, d), (4 * ld, 4)).copy()
+        enc = pkg.synthetic.bf16_round(x) if bf16 else x
+        first = shift + (T - 1) * -ld if ld < 0 else shift
+        got = _Rows(dev, enc, ld, shift + (T - 1) * abs(ld) + d, first)
+        return got, pkg.synthetic.bf16_to_f32(enc) if bf16 else x
+
+    (dq, q), (dk, k), (dv, v) = rows(ldq), rows(ldkv), rows(ldkv)
+    ref = orc.attention(q, k, v, cu, cu, heads)
+    seq = np.repeat(np.arange(len(lens), dtype=np.int32), lens)
+    out = dev.DeviceArray.zeros((T, d), np.float32)
+    dev.attention(dq, dk, dv, dev.DeviceArray.from_host(seq), dev.DeviceArray.from_host(cu), out, heads=heads,
+                  max_keys=int(max(lens)), bf16=bf16, head_dim=head_dim)
+    dev.synchronize()
+    assert np.array_equal(out.host().view(np.uint32), ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("M", [1, 64, 130])
 def test_vocab_argmax_matches_oracle(pkg, orc, dev, full_model, M):
     """Up to 64 rows one row group; 130 rows run three 64-row groups side
