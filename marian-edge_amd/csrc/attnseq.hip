@@ -263,6 +263,53 @@ __device__ __forceinline__ bool find_unit(const uint32_t* cu, int n, int heads, 
   return true;
 }
 
+// Rows q0, q0 + 1, ... of a sequence, past the query tiles of the launch: one
+// query per wave, lane = key or dimension, every operand straight from memory,
+// the arithmetic in the order above.  Only a sequence longer than max_keys said
+// comes here (the host does not know the lengths), so that its rows are written
+// all the same.
+template <int CH, typename T, int DH>
+__device__ __forceinline__ void rest_of_sequence(const AttnArgs& a, int64_t key0, int L, int Lc, int h, int q0, int w,
+                                                 int lane, float* sE, const uint64_t* sTab) {
+  const T* kh = (const T*)a.k + key0 * a.ldkv + h * DH;
+  const T* vh = (const T*)a.v + key0 * a.ldkv + h * DH + min(lane, DH - 1);
+  bool bad = false;
+#pragma unroll 1
+  for (int64_t r = q0 + w; r < L; r += kSeqWaves) {
+    const T* qr = (const T*)a.q + (key0 + r) * a.ldq + h * DH;
+    float mx = -INFINITY;
+#pragma unroll 1
+    for (int c = 0; c < CH && 64 * c < Lc; ++c) {
+      const T* kr = kh + min(64 * c + lane, Lc - 1) * a.ldkv;
+      float dot = -0.0f;
+#pragma unroll 1
+      for (int i = 0; i < DH; ++i) dot = dot + load1(qr + i) * load1(kr + i);
+      const float sc = 64 * c + lane < Lc ? dot * (1.0f / sqrtf((float)DH)) : -INFINITY;
+      sE[64 * c + lane] = sc;
+      mx = fmaxf(mx, sc);
+    }
+    mx = wave_max(mx);
+#pragma unroll 1
+    for (int c = 0; c < CH && 64 * c < Lc; ++c) sE[64 * c + lane] = ref_expf(sE[64 * c + lane] - mx, sTab);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's LDS writes land
+    __builtin_amdgcn_wave_barrier();
+    float sum = 0.0f, o = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < Lc; ++k) sum = sum + sE[k];
+    const float inv = 1.0f / sum;
+#pragma unroll 1
+    for (int k = 0; k < Lc; ++k) o = o + load1(vh + k * a.ldkv) * (sE[k] * inv);
+    __builtin_amdgcn_wave_barrier();
+    if (lane < DH) {
+      a.out[(key0 + r) * a.ldo + h * DH + lane] = o;
+      if (a.qout) a.qout[(key0 + r) * a.ldqout + h * DH + lane] = (int8_t)quantize_one(o, a.qmult);
+      bad |= !isfinite(o);
+    }
+    if (a.qout && h == 0 && lane == 0) a.qa[key0 + r] = a.qmult;
+  }
+  if (__any(bad) && lane == 0 && a.err) *a.err = 1;
+}
+
 // CH: 64-key chunks whose scores the registers hold (4: 256 keys; 8: 512 keys).
 // QW: queries per wave.
 // GEN: rows by 64-bit addresses, for the strides and alignments that
@@ -270,6 +317,7 @@ __device__ __forceinline__ bool find_unit(const uint32_t* cu, int n, int heads, 
 template <int CH, int QW, typename T, int DH, bool GEN>
 __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) void k_attn_seq(AttnArgs a) {
   static_assert(DH == 64 || DH == 48, "head widths");
+  static_assert(64 * CH <= 64 * kSeqRow / kSeqWaves, "a wave's part of the stage holds a query's scores");
   constexpr int W = kSeqWaves, TQ = W * QW;  // queries per workgroup
   constexpr int G = 64 / QW;                 // lane groups of a tile
   constexpr int NB = QW / 4;                 // tile blocks of 4 G rows
@@ -278,12 +326,13 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
   __shared__ __attribute__((aligned(16))) float sPall[TQ * kSeqRow];  // queries, then probabilities
   __shared__ uint64_t sTab[32];
   const int tid = threadIdx.x, lane = tid & 63;
-  int sq, qt, h0;
+  int sq, qt, h0, tiles;  // tiles: query tiles of the launch
   if (QW == 16 && a.n_seqs <= kSeqFindMax) {
     if (!find_unit<CH + 2>(a.cu, a.n_seqs, a.heads, blockIdx.x, lane, sq, qt, h0)) return;
     sq = __builtin_amdgcn_readfirstlane(sq);
     qt = __builtin_amdgcn_readfirstlane(qt);
     h0 = __builtin_amdgcn_readfirstlane(h0);
+    tiles = CH;  // the last class's
   } else {
     // Workgroups go round the XCDs in order: every sequence's heads lie on
     // different ones, but where short sequences' heads exit (below) the heads
@@ -291,7 +340,8 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
     const int x = blockIdx.x;
     sq = QW == 4 ? x / a.heads : x % a.n_seqs;
     h0 = QW == 4 ? x % a.heads : x / a.n_seqs;
-    qt = gridDim.y - 1 - blockIdx.y;  // high query tiles first
+    tiles = gridDim.y;
+    qt = tiles - 1 - blockIdx.y;  // high query tiles first
   }
   const int64_t key0 = a.cu[sq];
   const int L = (int)(a.cu[sq + 1] - key0);
@@ -483,6 +533,10 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
       if (a.qout && h == 0 && g == 0) a.qa[row] = a.qmult;
     }
     if (__any(bad) && lane == 0 && a.err) *a.err = 1;
+  }
+  if (L > tiles * TQ && qt == tiles - 1) {  // the whole workgroup
+    __syncthreads();  // the staged rows have been read
+    rest_of_sequence<CH, T, DH>(a, key0, L, Lc, h0, tiles * TQ, w, lane, stage + w * (64 * kSeqRow / W), sTab);
   }
 }
 

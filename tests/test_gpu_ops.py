@@ -655,6 +655,40 @@ def test_packed_attention_row_strides(pkg, orc, dev, heads, head_dim, bf16, lens
     assert np.array_equal(out.host().view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("heads,head_dim,bf16,lens,max_keys", [
+    (4, 64, False, [150, 40, 16, 3], 100), (4, 48, True, [150, 40, 16, 256], 1), (2, 64, False, [500, 3, 300], 300),
+    (8, 64, False, [200] * 30, 100), (4, 48, True, [40, 200] * 50, 20),
+    (2, 64, False, [1 + (11 * i) % 70 for i in range(1030)], 20),
+    # longer than the launch holds scores for: the first 256 (512) keys
+    (4, 64, False, [300, 20, 257], 200), (8, 48, True, [300, 20] * 20, 200), (2, 64, True, [600, 20], 400),
+    (4, 64, False, [600, 20] * 16, 400),
+])
+def test_packed_attention_understated_max_keys(pkg, orc, dev, heads, head_dim, bf16, lens, max_keys):
+    """Sequences longer than max_keys: every row is written, over all its keys up to
+    256 (512 with max_keys above 256), bit-identical to the oracle."""
+    print(f"packed attention heads={heads} head_dim={head_dim} bf16={bf16} max_keys={max_keys}", flush=True)
+    rng = np.random.default_rng(47)
+    d, T = heads * head_dim, sum(lens)
+    hold = 256 if max_keys <= 256 else 512
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    seq = np.repeat(np.arange(len(lens), dtype=np.int32), lens)
+    first = np.arange(T) - cu[seq].astype(np.int64) < hold  # keys that count
+    cu_k = np.concatenate([[0], np.cumsum(np.minimum(lens, hold))]).astype(np.uint32)
+    q, k, v = (rng.standard_normal((T, d)).astype(np.float32) for _ in range(3))
+    if bf16:
+        enc = [pkg.synthetic.bf16_round(x) for x in (q, k, v)]
+        q, k, v = (pkg.synthetic.bf16_to_f32(x) for x in enc)
+    else:
+        enc = [q, k, v]
+    ref = orc.attention(q, np.ascontiguousarray(k[first]), np.ascontiguousarray(v[first]), cu, cu_k, heads)
+    out = dev.DeviceArray(ref.shape, np.float32)
+    out.fill_bytes(0xFF)
+    dev.attention(*(dev.DeviceArray.from_host(x) for x in enc), dev.DeviceArray.from_host(seq),
+                  dev.DeviceArray.from_host(cu), out, heads=heads, max_keys=max_keys, bf16=bf16, head_dim=head_dim)
+    dev.synchronize()
+    assert np.array_equal(out.host().view(np.uint32), ref.view(np.uint32))
+
+
 @pytest.mark.parametrize("M", [1, 64, 130])
 def test_vocab_argmax_matches_oracle(pkg, orc, dev, full_model, M):
     """Up to 64 rows one row group; 130 rows run three 64-row groups side
