@@ -56,6 +56,12 @@ constexpr int kSeqWaves = 4;                   // waves per workgroup
 // 4363 62.9 | 59.0; 257-512 keys, 1325 rows 48.3 | 71.1, 2431 78.2 | 78.8, 4290
 // 110 | 106).
 constexpr int64_t kSeqFewRows256 = 32768, kSeqFewRows512 = 20480;
+// Workgroups up to which that holds: max_keys may be far above the lengths, and
+// each 4096 that find nothing cost 0.9 us, where with 16 queries the lengths
+// decide (1024 sequences of 4 rows, max_keys 4: 8192 workgroups, 25.5 us with 4
+// queries | 44.0 with 16; max_keys 256: 131072, 52.9 | 44.0; 300 of 8 rows,
+// 38400: 20.6 | 15.1; 90 sentences, 23040: 22.3 | 22.7).
+constexpr int64_t kSeqFewGroups = 24576;
 constexpr int kSeqFindMax = 1024;              // sequences up to which a workgroup finds its unit itself
 constexpr int kSeqRow = kHeadDim + 4;          // padded LDS row (floats), 16-byte aligned
 
@@ -571,7 +577,8 @@ hipError_t launch_attention_seq(const AttnArgs& a, hipStream_t s) {
       (int64_t)a.n_seqs * a.heads > 0x7fffffff || (int64_t)a.rows * a.heads > 0x7fffffff)
     return hipErrorInvalidValue;
   const bool gen = !seq_buffer_rows(a);
-  const bool few = !gen && (int64_t)a.rows * a.heads <= (a.max_keys <= 256 ? kSeqFewRows256 : kSeqFewRows512);
+  const bool few = !gen && (int64_t)a.rows * a.heads <= (a.max_keys <= 256 ? kSeqFewRows256 : kSeqFewRows512) &&
+                   (int64_t)a.n_seqs * a.heads * ((a.max_keys + 4 * kSeqWaves - 1) / (4 * kSeqWaves)) <= kSeqFewGroups;
   const int tq = kSeqWaves * (few ? 4 : 16);
   // Units: at most heads / 4 + 7 / 256 heads L of a sequence of L rows (equal at 65 rows).
   const int64_t units = (int64_t)a.n_seqs * ((a.heads + 3) / 4) + ((int64_t)a.rows * a.heads * 7 + 255) / 256;

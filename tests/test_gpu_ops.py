@@ -662,10 +662,12 @@ def test_packed_attention_row_strides(pkg, orc, dev, heads, head_dim, bf16, lens
     # longer than the launch holds scores for: the first 256 (512) keys
     (4, 64, False, [300, 20, 257], 200), (8, 48, True, [300, 20] * 20, 200), (2, 64, True, [600, 20], 400),
     (4, 64, False, [600, 20] * 16, 400),
+    # far above the lengths: launches of many workgroups without a query
+    (8, 64, False, [3, 17] * 120, 256), (8, 48, True, [1, 40] * 45, 512), (4, 64, False, [1, 4, 7] * 400, 256),
 ])
-def test_packed_attention_understated_max_keys(pkg, orc, dev, heads, head_dim, bf16, lens, max_keys):
-    """Sequences longer than max_keys: every row is written, over all its keys up to
-    256 (512 with max_keys above 256), bit-identical to the oracle."""
+def test_packed_attention_max_keys_off_the_lengths(pkg, orc, dev, heads, head_dim, bf16, lens, max_keys):
+    """Sequences longer than max_keys (every row is written, over all its keys up to
+    256, or 512 with max_keys above 256) or much shorter: bit-identical to the oracle."""
     print(f"packed attention heads={heads} head_dim={head_dim} bf16={bf16} max_keys={max_keys}", flush=True)
     rng = np.random.default_rng(47)
     d, T = heads * head_dim, sum(lens)
