@@ -98,19 +98,23 @@ def test_q8_linear_tile_sizes(dev, M, K, N):
     acc = (q.astype(dt) @ w.astype(dt).T).astype(np.int32)
     D = dev.DeviceArray
     dq, dw, da, dm, db = (D.from_host(x) for x in (q, w, a, mult, bias))
-    di, df = D.zeros((M, N), np.int32) if N < 4096 else None, D.zeros((M, N), np.float32)
+    di, df = D.zeros((M, N), np.int32), D.zeros((M, N), np.float32)
     for relu in (False, True) if N < 4096 else (False,):
         want = _dequant_ref(acc, a, mult, bias, relu)
         df.fill_bytes(0xFF)
         dev.q8_linear(None, dw, dm, db, None, df, relu=relu, xq=dq, xa=da)
         dev.synchronize()
         assert np.array_equal(df.host().view(np.uint32), want.view(np.uint32)), f"fp32 relu={relu}"
-        if di is not None:
-            df.fill_bytes(0xFF)
-            dev.q8_linear(None, dw, dm, db, di, df, relu=relu, xq=dq, xa=da)
-            dev.synchronize()
-            assert np.array_equal(di.host(), acc)
-            assert np.array_equal(df.host().view(np.uint32), want.view(np.uint32)), f"both relu={relu}"
+        df.fill_bytes(0xFF)
+        di.fill_bytes(0xFF)
+        dev.q8_linear(None, dw, dm, db, di, df, relu=relu, xq=dq, xa=da)
+        dev.synchronize()
+        assert np.array_equal(di.host(), acc)
+        assert np.array_equal(df.host().view(np.uint32), want.view(np.uint32)), f"both relu={relu}"
+    di.fill_bytes(0xFF)
+    dev.q8_linear(None, dw, dm, db, di, None, xq=dq, xa=da)
+    dev.synchronize()
+    assert np.array_equal(di.host(), acc), "int32 alone"
 
 
 @pytest.mark.parametrize("M,K,N", [

@@ -92,6 +92,24 @@ def test_ssru_probe_bit_exact(pkg, orc, step):
     assert np.array_equal(lg[act_o].view(np.uint32), lg_o[act_o].view(np.uint32))
 
 
+def test_ssru_encoder_of_many_rows_bit_exact(pkg, orc):
+    """2600 packed rows: the encoder's FFN runs on the 128x128 tiles of the
+    many-row GEMM, which also store the next layer's int8 codes."""
+    g = pkg.SsruGeometry(source_vocab=3000, target_vocab=3200, encoder_layers=2, decoder_layers=1)
+    model = pkg.seeded_ssru_model(seed=43, geometry=g, std=0.05)
+    om = orc.OracleSsruModel(model)
+    rng = np.random.default_rng(17)
+    seqs = [rng.integers(3, g.source_vocab, size=130).astype(np.int32) for _ in range(20)]
+    b = pkg.synthetic._pack("rows", seqs, [1] * 20, 0, dict(pkg.synthetic.LIFTED_LIMITS))
+    with pkg.HipEngine(model, limits=b.limits) as e:
+        out, enc, _, _ = e.translate_probe(b.tokens, b.offsets, b.max_output_tokens, pkg.FLAG_IGNORE_EOS, probe_step=0)
+    rows, enc_o, _, _ = orc.translate_ssru(om, b.tokens, b.offsets, b.max_output_tokens, b.limits,
+                                           pkg.FLAG_IGNORE_EOS, probe_step=0, threads=ORACLE_THREADS)
+    print(f"{b.tokens.size} rows", flush=True)
+    assert out.rows() == rows
+    assert np.array_equal(enc.view(np.uint32), enc_o.view(np.uint32))
+
+
 def test_ssru_long_sentences_token_exact(pkg, orc):
     """Sentences longer than 128 tokens and an FFN width that is not a
     multiple of 128: every step's SSRU LayerNorm, query projection and
