@@ -115,10 +115,11 @@ __device__ __forceinline__ void tile_pass(__amdgpu_buffer_rsrc_t r, int64_t ld, 
 // Dequantizes and stores one wave's blocks of a tile at (m0, n0): rows wr +
 // 32 i, columns wc + 32 k.  sAm: the tile's row multipliers in LDS; ok: this
 // lane's share of them has exponents in recip_exact's range.
+// stream: the fp32 and int32 stores are non-temporal.
 template <int BM, int MB, int NB, bool RELU, bool EXTRA, bool WIDE>
 __device__ __forceinline__ void tile_store(const GemmArgs& g, const Epilogue& e, const v16i (&acc)[MB][NB],
                                            const float* sAm, const float (&wm)[NB], const float (&bi)[NB], bool ok,
-                                           int m0, int n0, int wr, int wc) {
+                                           int m0, int n0, int wr, int wc, bool stream) {
   const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5;
 #pragma unroll
   for (int k = 0; k < NB; ++k) ok &= recip_factor(wm[k]);
@@ -153,7 +154,10 @@ __device__ __forceinline__ void tile_store(const GemmArgs& g, const Epilogue& e,
   } else {
     auto pass = [&](auto out, const void* p, int64_t ld) {
       const __amdgpu_buffer_rsrc_t r = tile_rows(p, m0 * ld, ld, rows, 4);
-      tile_pass<out(), kNt, RELU>(r, ld, g, acc, sm, wm, bi, ok, row0, ncol, 0.0f, rows, bad);
+      if (stream)
+        tile_pass<out(), kNt, RELU>(r, ld, g, acc, sm, wm, bi, ok, row0, ncol, 0.0f, rows, bad);
+      else
+        tile_pass<out(), 0, RELU>(r, ld, g, acc, sm, wm, bi, ok, row0, ncol, 0.0f, rows, bad);
     };
     if (!EXTRA || e.out) pass(std::integral_constant<TileOut, TO_F32>(), e.out, e.ldo);
     if constexpr (EXTRA) {
@@ -173,7 +177,7 @@ __device__ __forceinline__ void tile_store(const GemmArgs& g, const Epilogue& e,
 
 template <int BM, int BN, int WM, int WN, int PF, bool RELU, bool EXTRA, bool WIDE>
 __global__ __launch_bounds__(WM * WN * 64) __attribute__((amdgpu_waves_per_eu(BM > 128 ? 2 : WM * WN / 2)))
-void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
+void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles, int stream) {
   constexpr int NT = WM * WN * 64;
   constexpr int MB = BM / WM / 32, NB = BN / WN / 32;  // 32x32 blocks per wave
   constexpr int AP = BM * 8 / NT, BP = BN * 8 / NT;    // 16-byte pieces per thread and chunk
@@ -298,7 +302,7 @@ void k_gemm_tile(GemmArgs g, Epilogue e, int tiles_n, int tiles) {
     bool ok = true;
 #pragma unroll
     for (int i = 0; i < BM; i += 64) ok &= recip_factor(sAm[tpar][i + lane]);
-    tile_store<BM, MB, NB, RELU, EXTRA, WIDE>(g, e, acc, sAm[tpar], wm, bi, ok, m0, n0, wr, wc);
+    tile_store<BM, MB, NB, RELU, EXTRA, WIDE>(g, e, acc, sAm[tpar], wm, bi, ok, m0, n0, wr, wc, stream);
     m0 = m1;
     n0 = n1;
   }
@@ -434,7 +438,23 @@ __global__ __launch_bounds__(WM * WN * 64) void k_gemm_tile_f32(GemmArgs g, Epil
       }
     }
   }
-  tile_store<BM, MB, NB, RELU, EXTRA, false>(g, e, acc, sAm, wm, bi, recip_factor(sAm[lane]), m0, n0, wr, wc);
+  tile_store<BM, MB, NB, RELU, EXTRA, false>(g, e, acc, sAm, wm, bi, recip_factor(sAm[lane]), m0, n0, wr, wc, true);
+}
+
+// Whether the outputs are stored past the caches.  Rows of whole 64-byte pieces
+// are (16384 x 2304, K = 512: 41.1 us, 60.2 through the caches).  In other rows a
+// store instruction ends inside a piece at either end, and streaming the parts
+// costs more than leaving them to the caches to join, once the outputs exceed
+// the L2s and as long as the last cache holds them beside the operands, or the
+// products are few (us; streamed | not, before this kernel): 2200 x 2300, K 512
+// 11.1 | 12.1, 13.3; 8192 x 2300, K 256 32.2 | 22.1, 26.7; 3000 x 8300, K 512 54.5 |
+// 36.0, 46.7; 16384 x 1500, K 512 40.3 | 44.0, 44.7; 16384 x 1000, K 2048 54.0 | 59.6.
+// With both outputs streaming never paid (4096 x 8300, K 512 153 | 99, 114).
+bool tile_streams(const GemmArgs& g, const Epilogue& e) {
+  const bool whole = ((e.out ? (uintptr_t)e.out | 4 * e.ldo : 0) | (e.out_i32 ? (uintptr_t)e.out_i32 | 4 * e.ldi : 0)) % 64 == 0;
+  if (e.out && e.out_i32) return whole;
+  const int64_t mb = (int64_t)g.M * g.N * 4 / 1000000;
+  return whole || mb < 26 || (g.K > 256 && mb > (g.K > 512 ? 60 : (g.N > kTileWideN * 128 ? 128 : 88)));
 }
 
 template <int BM, int BN, int WM, int WN, int PF, bool WIDE = false>
@@ -445,7 +465,8 @@ hipError_t launch_tile(const GemmArgs& g, const Epilogue& e, int max_wgs, hipStr
   const bool extra = WIDE || e.out_i32 || e.out_q || !e.out;
   auto kern = e.relu ? (extra ? k_gemm_tile<BM, BN, WM, WN, PF, true, true, WIDE> : k_gemm_tile<BM, BN, WM, WN, PF, true, WIDE, WIDE>)
                      : (extra ? k_gemm_tile<BM, BN, WM, WN, PF, false, true, WIDE> : k_gemm_tile<BM, BN, WM, WN, PF, false, WIDE, WIDE>);
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(WM * WN * 64), 0, s, g, e, (int)tiles_n, (int)tiles);
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(WM * WN * 64), 0, s, g, e, (int)tiles_n, (int)tiles,
+                     (int)tile_streams(g, e));
   return hipGetLastError();
 }
 
@@ -477,10 +498,13 @@ hipError_t launch_gemm_tile(const GemmArgs& g, const Epilogue& e, hipStream_t s)
   //     1459 x 512 (K 512) 5.1 / 6.9 / 9.3, 4096 x 512 (K 2048) 12.0 / 14.1 / 19.8;
   //   above, larger tiles read less per output: 7405 x 512 (K 2048) 17.8 / 14.4 /
   //     19.3, 1000 x 32000 44.9 / 34.0 / 36.9;
+  //   past one round of 128x128 tiles their outputs count without the padding:
+  //     12000 x 300 (K 2048; 282 tiles, 220 without) 20.0 / 24.4;
   //   from 2048 256x128 tiles (eight a CU) the largest: 4096 x 32000 175 / 157 / 134.
   const auto tiles = [&](int64_t bm, int64_t bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
+  const bool one_round = tiles(128, 128) >= 224 && tiles(128, 128) <= 256;
   if (tiles(256, 128) >= 2048) return launch_tile<256, 128, 4, 2, 2>(g, e, 256, s);
-  if (tiles(128, 128) >= 224) return launch_tile<128, 128, 2, 4, 2>(g, e, 1 << 30, s);
+  if (one_round || (int64_t)g.M * g.N >= 224 * 128 * 128) return launch_tile<128, 128, 2, 4, 2>(g, e, 1 << 30, s);
   return launch_tile<64, 64, 2, 2, 2>(g, e, 1024, s);
 }
 

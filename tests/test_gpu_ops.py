@@ -78,6 +78,8 @@ def _dequant_ref(acc, a, mult, bias, relu=False):
     (1793, 320, 2047), (1920, 128, 1900),                   # 128x128 tiles: from 224 of them
     (2305, 64, 29057),                                      # 256x128 tiles: from 2048, the last row tile of one row
     (65, 64, (1 << 20) + 8),                                # output rows past the buffer stores' offsets
+    (7001, 64, 1001), (3600, 512, 2050),                    # rows stored through the caches: over 26 MB, odd strides
+    (20001, 64, 150),                                       # past a round of padded 128x128 tiles: 64x64
 ])
 def test_q8_linear_tile_sizes(dev, M, K, N):
     """Every tile size of the many-row GEMM at its edges, bit-identical to the
