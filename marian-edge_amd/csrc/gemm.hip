@@ -816,9 +816,22 @@ hipError_t launch_vocab_argmax(const GemmArgs& g, const Epilogue& e, hipStream_t
 // workgroups per row group (64 x 32000: 19 us against 7.8 on row tiles).
 static bool linear_f32_skinny(const GemmArgs& g) { return g.M <= kSkinnyRows && (g.M <= kAfRows || g.N < 8192); }
 
+// The repeated quantization grows with K: above 512 a launch of more than one
+// round of workgroups (two of 16 waves fit a CU, one of them with two k-steps a
+// wave, above 1024) is slower than quantizing first (us in one launch | two: 64 x
+// 2048, K = 2048 9.8 | 11.4; 64 x 2300 17.2 | 11.7; 33 x 6000, K = 1536 18.7 | 12.2;
+// 64 x 4000, K = 1024 9.7 | 13.1; 33 x 6000, K = 768, 564 workgroups 9.8 | 11.0; 49 x
+// 8000 13.9 | 11.7).  Up to 16 rows only K = 2048 gets there, whose rows quantize
+// fastest by themselves (16 x 32000 22.9 | 20.0; K = 1536 21.3 | 34.5).
+static bool linear_f32_one_round(const GemmArgs& g) {
+  const int64_t groups = (int64_t)skinny_groups(g.N) * ((g.M + kAfRows - 1) / kAfRows);
+  if (g.M <= kAfRows) return g.K < kSkinnyMaxK || groups <= 256;
+  return g.K <= 512 || groups <= (g.K <= 1024 ? 576 : 256);
+}
+
 bool linear_f32_fused(const GemmArgs& g, const Epilogue& e) {
   if (!g.Af || g.Aamax || g.M_dev || e.out_q || g.ldaf % 4 || (uintptr_t)g.Af % 16) return false;
-  return linear_f32_skinny(g) ? g.K <= kSkinnyMaxK : gemm_f32_supported(g, e);
+  return linear_f32_skinny(g) ? g.K <= kSkinnyMaxK && linear_f32_one_round(g) : gemm_f32_supported(g, e);
 }
 
 hipError_t launch_linear_f32(const GemmArgs& g, const Epilogue& e, hipStream_t s) {

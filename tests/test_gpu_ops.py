@@ -124,6 +124,8 @@ def test_q8_linear_tile_sizes(dev, M, K, N):
     (17, 512, 8200), (64, 64, 9000), (65, 192, 127), (129, 512, 1000),  # row tiles, 128 columns
     (1100, 320, 2300),                                                  # row tiles, 256 columns
     (65, 576, 64), (5000, 512, 2048),                                   # quantized first
+    (64, 1536, 2300), (33, 1024, 8100), (16, 2048, 20000),              # quantized first: past one round of workgroups
+    (64, 1536, 2048), (32, 1024, 8100), (16, 1984, 20000),              # and not
 ])
 @pytest.mark.parametrize("act", [0.0, 31.75])
 def test_q8_linear_from_fp32_rows(dev, M, K, N, act):
