@@ -174,9 +174,14 @@ __global__ __launch_bounds__(256) void k_residual_ln(const float* y, const float
 // 18.9 -> 15.6; 7405 rows of 256 8.65 -> 8.18, of 384 11.2 -> 10.8, of 512 13.1 ->
 // 13.4; 16384 rows of 256 14.6 -> 12.1, of 384 19.0 -> 15.4, of 512 25.4 -> 25.2.
 // Fewer rows leave the chip idle and the longer chains show (4500 rows of 384
-// 8.25 -> 9.80; 1459 of 1024 11.9 -> 15.2).
-template <int PER>
-constexpr int kLnManyRows = PER == 8 ? INT32_MAX : (kLnSpec<PER> ? 7168 : 2560);
+// 8.25 -> 9.80; 1459 of 1024 11.9 -> 15.2), and a third round of 4096 rows has to
+// be filled for a third before it pays (8656 rows of 384 12.05 -> 12.65, of 256
+// 9.41 -> 9.75; 9472 of 384 13.5 -> 13.3).
+bool ln_many_rows(int d, int rows) {
+  if (d == 512) return false;
+  if (d == 256 || d == 384) return rows >= 9472 || (rows >= 7168 && rows <= 8192);
+  return rows >= 2560;
+}
 template <int PER>
 constexpr int kLnR = PER <= 8 ? 4 : 2;
 template <int V>
@@ -717,12 +722,15 @@ hipError_t launch_quantize_rows(const float* x, int64_t ldx, int rows, const int
   }
 
 template <int PER>
-static void launch_ln_rows(const float* y, const float* r, const float* g, const float* b, int rows, float* out,
-                           int8_t* q, float* a, int* err, hipStream_t s) {
-  if constexpr (PER != 8) {  // rows of 512 keep one wave each
+static hipError_t launch_ln_rows(const float* y, const float* r, const float* g, const float* b, int rows, float* out,
+                                 int8_t* q, float* a, int* err, hipStream_t s) {
+  if constexpr (PER == 8) {
+    return hipErrorInvalidValue;  // rows of 512 keep one wave each (ln_many_rows)
+  } else {
     constexpr int R = kLnR<PER>;
     hipLaunchKernelGGL((k_residual_ln_rows<PER, R>), dim3((rows + 4 * R - 1) / (4 * R)), dim3(256), 0, s, y, r, g, b,
                        rows, out, q, a, err);
+    return hipGetLastError();
   }
 }
 hipError_t launch_residual_ln(const float* y, const float* r, const float* g, const float* b,
@@ -730,18 +738,18 @@ hipError_t launch_residual_ln(const float* y, const float* r, const float* g, co
                               float* a, int* err, hipStream_t s, float qmult, bool fast) {
   if (rows <= 0) return hipSuccess;
   if (d % 64) return hipErrorInvalidValue;
-  // Many rows: several per wave.  Else one wave per row, four rows per workgroup: widths of 256, 384 and 512
-  // fold with the one-wave speculative folds, others sequentially; with
-  // `fast` (the decoder's widths) the sums take the tree order.
+  // Many rows: several per wave.  Else one wave per row, four rows per
+  // workgroup: widths of 256, 384 and 512 fold with the one-wave speculative
+  // folds, others sequentially; with `fast` (the decoder's widths) the sums take
+  // the tree order.
   const dim3 grid((rows + 3) / 4), block(256);
 #define MH_LN(P) \
   hipLaunchKernelGGL(k_residual_ln<P>, grid, block, 0, s, y, r, g, b, rows, rows_dev, out, q, a, err, qmult)
 #define MH_LNF(P)                                                                                            \
   hipLaunchKernelGGL((k_residual_ln<P, true>), grid, block, 0, s, y, r, g, b, rows, rows_dev, out, q, a, err, \
                      qmult)
-  const int many = d == 512 ? kLnManyRows<8> : (d == 256 || d == 384 ? kLnManyRows<4> : kLnManyRows<1>);
-  if (!fast && !rows_dev && !(qmult > 0.0f) && rows >= many) {
-#define MH_LNR(P) launch_ln_rows<P>(y, r, g, b, rows, out, q, a, err, s)
+  if (!fast && !rows_dev && !(qmult > 0.0f) && ln_many_rows(d, rows)) {
+#define MH_LNR(P) return launch_ln_rows<P>(y, r, g, b, rows, out, q, a, err, s)
     MH_PER_DISPATCH_16(d / 64, MH_LNR)
   } else if (fast) {
     MH_PER_DISPATCH(d / 64, MH_LNF)

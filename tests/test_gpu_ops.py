@@ -333,11 +333,13 @@ def test_residual_layer_norm_matches_oracle(pkg, orc, dev):
         assert np.array_equal(q.host(), q_ref) and np.array_equal(a.host(), a_ref)
 
 
-@pytest.mark.parametrize("d,rows", [(64, 2560), (192, 2561), (256, 7168), (256, 7171), (384, 7169), (512, 7405),
-                                    (640, 2563), (960, 2561), (1024, 2562)])
+@pytest.mark.parametrize("d,rows", [(64, 2560), (192, 2561), (256, 7168), (256, 7171), (384, 7169), (384, 9473),
+                                    (640, 2563), (960, 2561), (1024, 2562),
+                                    (512, 7405), (256, 8193), (384, 9471)])  # one row per wave
 def test_residual_layer_norm_many_rows(pkg, orc, dev, d, rows):
-    """Several rows per wave: every width's lane layout, a last wave with fewer
-    rows, rows that start at any float, and non-finite rows."""
+    """Several rows per wave at every lane layout (512 and a few row counts keep one
+    row per wave): a last wave with fewer rows, rows that start at any float, and
+    non-finite rows."""
     print(f"residual_layer_norm {rows} x {d}", flush=True)
     rng = np.random.default_rng(29)
     y = rng.standard_normal((rows, d)).astype(np.float32)
