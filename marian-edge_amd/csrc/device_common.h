@@ -84,13 +84,6 @@ __device__ __forceinline__ float xor_lane_f(float v) {
   return __int_as_float(xor_lane<OFF>(__float_as_int(v)));
 }
 
-template <int OFF>
-__device__ __forceinline__ uint64_t xor_lane_u64(uint64_t v) {
-  const uint32_t lo = (uint32_t)xor_lane<OFF>((int)(uint32_t)v);
-  const uint32_t hi = (uint32_t)xor_lane<OFF>((int)(uint32_t)(v >> 32));
-  return ((uint64_t)hi << 32) | lo;
-}
-
 // Maximum over the wave; max is exact in any order, so the reduction uses
 // VALU-only lane moves: DPP within each 16-lane row (quad swaps, rotations by
 // 4 and 8), then the four row maxima are read out as scalars.  Every lane
@@ -118,16 +111,6 @@ __device__ __forceinline__ uint32_t row16_max(uint32_t p) {
   p = max(p, (uint32_t)dpp_mov<0x4E>((int)p));   // quad_perm [2,3,0,1]
   p = max(p, (uint32_t)dpp_mov<0x124>((int)p));  // row_ror:4
   return max(p, (uint32_t)dpp_mov<0x128>((int)p));  // row_ror:8
-}
-
-// Maximum over each 32-lane half of the wave (every lane returns its half's):
-// the row maxima by DPP, then rows 0-1 and 2-3 paired by a lane swap.
-__device__ __forceinline__ float half_wave_max(float p) {
-  p = fmaxf(p, __int_as_float(dpp_mov<0xB1>(__float_as_int(p))));   // quad_perm [1,0,3,2]
-  p = fmaxf(p, __int_as_float(dpp_mov<0x4E>(__float_as_int(p))));   // quad_perm [2,3,0,1]
-  p = fmaxf(p, __int_as_float(dpp_mov<0x124>(__float_as_int(p))));  // row_ror:4
-  p = fmaxf(p, __int_as_float(dpp_mov<0x128>(__float_as_int(p))));  // row_ror:8
-  return fmaxf(p, xor_lane_f<16>(p));
 }
 
 __device__ __forceinline__ uint64_t umax64(uint64_t a, uint64_t b) { return a > b ? a : b; }
@@ -462,8 +445,9 @@ __device__ __forceinline__ float row_multiplier(float absmax) {
 
 // 1 / x for a positive x in [2^-125, 2^126): the hardware's estimate and one
 // Newton step.  Equal to the IEEE quotient on every float of that range (all
-// 2^31 of them compared on the device), three instructions instead of the
-// division's ten.
+// 251 * 2^23 of them compared on the device once; test_q8_linear_reciprocals
+// compares every mantissa at the range's ends and in its middle), three
+// instructions instead of the division's ten.
 __device__ __forceinline__ float recip_exact(float x) {
   const float r = __builtin_amdgcn_rcpf(x);
   return __builtin_fmaf(__builtin_fmaf(-x, r, 1.0f), r, r);

@@ -119,6 +119,65 @@ def test_q8_linear_tile_sizes(dev, M, K, N):
     assert np.array_equal(di.host(), acc), "int32 alone"
 
 
+def test_q8_linear_reciprocals(dev):
+    """The dequantization's 1 / (a w) where it is taken without a division: every
+    mantissa at both ends of the factors' range and in its middle."""
+    M, K, D = 1 << 20, 64, dev.DeviceArray
+    q, w = np.zeros((M, K), np.int8), np.zeros((3, K), np.int8)
+    q[:, 0], w[:, 0] = 1, 1  # every accumulator is 1
+    mult = np.float32(2.0) ** np.array([-62, 0, 61], np.float32)
+    dq, dw, dm, db = (D.from_host(v) for v in (q, w, mult, np.zeros(3, np.float32)))
+    out = D.zeros((M, 3), np.float32)
+    for ea in (-62, 0, 61):
+        print(f"reciprocals 2^{ea}", flush=True)
+        for first in range(0, 1 << 23, M):
+            a = (((ea + 127) << 23) + first + np.arange(M, dtype=np.uint32)).astype(np.uint32).view(np.float32)
+            da = D.from_host(a)
+            dev.q8_linear(None, dw, dm, db, None, out, xq=dq, xa=da)
+            dev.synchronize()
+            want = np.float32(1) / (a[:, None] * mult[None, :])
+            assert want.dtype == np.float32
+            assert np.array_equal(out.host().view(np.uint32), want.view(np.uint32)), (ea, first)
+
+
+@np.errstate(over="ignore")
+def test_reciprocal_factor_limits(dev):
+    """Multipliers at the first and last float for which the division is left out,
+    and right outside them, in each kernel that does so: IEEE results either side."""
+    K, N, D = 64, 64, dev.DeviceArray
+    lo, hi = np.float32(2.0) ** np.float32(-62), np.float32(2.0) ** np.float32(62)
+    edges = [np.nextafter(lo, np.float32(0)), lo, np.float32(1.7), np.nextafter(hi, np.float32(0)), hi]
+    rng = np.random.default_rng(57)
+    q = rng.integers(-127, 128, (65, K)).astype(np.int8)
+    w = rng.integers(-127, 128, (N, K)).astype(np.int8)
+    bias = np.zeros(N, np.float32)
+    acc = (q.astype(np.int32) @ w.astype(np.int32).T).astype(np.float32)
+    dq, dw, db = (D.from_host(v) for v in (q, w, bias))
+    out, tok = D.zeros((65, N), np.float32), D.zeros(65, np.int32)
+    for a in edges:
+        da = D.from_host(np.full(65, a, np.float32))
+        for m in edges:
+            dm = D.from_host(np.full(N, m, np.float32))
+            want = acc * (np.float32(1) / (np.float32(a) * np.float32(m))) + bias
+            dev.q8_linear(None, dw, dm, db, None, out, xq=dq, xa=da)
+            dev.synchronize()
+            assert np.array_equal(out.host().view(np.uint32), want.view(np.uint32)), ("rows of int8", a, m)
+            # fp32 rows that the static multiplier a takes back to q (up to their rounding)
+            x = (q.astype(np.float64) / np.float64(a)).astype(np.float32)
+            xq = np.clip(np.rint(x * np.float32(a)), -127, 127)
+            ws = (xq.astype(np.int32) @ w.astype(np.int32).T).astype(np.float32)
+            dev.q8_linear_static(D.from_host(x), float(a), dw, dm, db, None, out)
+            dev.synchronize()
+            sw = ws * (np.float32(1) / (np.float32(a) * np.float32(m))) + bias
+            assert np.array_equal(out.host().view(np.uint32), sw.view(np.uint32)), ("fp32 rows", a, m)
+            dev.vocab_argmax(dq, da, dw, dm, db, tok, logits=out)
+            dev.synchronize()
+            lg = want.copy()
+            lg[:, [1, *range(7, 39)]] = -np.inf
+            assert np.array_equal(out.host().view(np.uint32), lg.view(np.uint32)), ("vocabulary", a, m)
+            assert np.array_equal(tok.host(), lg.argmax(1))
+
+
 @pytest.mark.parametrize("M,K,N", [
     (1, 64, 33), (16, 448, 100), (17, 512, 96), (64, 1024, 1030), (61, 1536, 384), (3, 2048, 70),  # 16-row groups
     (17, 512, 8200), (64, 64, 9000), (65, 192, 127), (129, 512, 1000),  # row tiles, 128 columns
@@ -600,6 +659,37 @@ def test_packed_attention_units(pkg, orc, dev, heads, head_dim, bf16, lens):
     assert np.all(got[:, d] == 0.0)
     got = np.ascontiguousarray(got[:, :d])
     nan = np.isnan(ref)
+    assert np.array_equal(nan, np.isnan(got))
+    assert np.array_equal(np.where(nan, 0, got).view(np.uint32), np.where(nan, 0, ref).view(np.uint32))
+
+
+@pytest.mark.parametrize("heads,head_dim,lens", [(8, 64, [200, 3, 31] * 12), (8, 64, [17, 200]), (4, 48, [500, 40])])
+def test_packed_attention_products(pkg, orc, dev, heads, head_dim, lens):
+    """The products come from the matrix cores.  With one non-zero value row per
+    sequence an output is one product, rounded by itself: values of every bit
+    pattern (denormal, infinite, NaN, both zeros) times probabilities down to
+    denormals, bit for bit against the oracle."""
+    print(f"packed attention products heads={heads} lens={len(lens)}", flush=True)
+    rng = np.random.default_rng(53)
+    d, T = heads * head_dim, sum(lens)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.uint32)
+    seq = np.repeat(np.arange(len(lens), dtype=np.int32), lens)
+    q, k = (rng.standard_normal((T, d)).astype(np.float32) * np.float32(s) for s in (6.0, 3.0))
+    v = np.zeros((T, d), np.float32)
+    at = cu[:-1].astype(np.int64) + rng.integers(0, lens)
+    v[at] = rng.integers(0, 1 << 32, (len(lens), d), dtype=np.uint32).view(np.float32)
+    v[at, ::5] = rng.integers(0, 1 << 24, (len(lens), v[0, ::5].size), dtype=np.uint32).view(np.float32)  # small
+    v[at, 1::9], v[at, 2::9], v[at, 3::9] = np.inf, -0.0, np.nan
+    with np.errstate(all="ignore"):
+        ref = orc.attention(q, k, v, cu, cu, heads)
+    out = dev.DeviceArray.zeros((T, d), np.float32)
+    dev.attention(*(dev.DeviceArray.from_host(x) for x in (q, k, v)), dev.DeviceArray.from_host(seq),
+                  dev.DeviceArray.from_host(cu), out, heads=heads, max_keys=max(lens), head_dim=head_dim)
+    dev.synchronize()
+    got, nan = out.host(), np.isnan(ref)
+    small = (ref != 0) & (np.abs(ref) < np.finfo(np.float32).tiny)
+    print(f"{ref.size} products, {int(small.sum())} denormal, {int(nan.sum())} NaN", flush=True)
+    assert small.any() and nan.any() and np.isinf(ref).any()
     assert np.array_equal(nan, np.isnan(got))
     assert np.array_equal(np.where(nan, 0, got).view(np.uint32), np.where(nan, 0, ref).view(np.uint32))
 
