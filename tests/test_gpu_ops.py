@@ -286,39 +286,69 @@ def test_q8_linear_outputs_over_the_input(dev, M, K, N, act):
                 assert np.array_equal(out.host().view(np.uint32), want.host().view(np.uint32)), (first_in, first_out, ints)
 
 
-def test_q8_linear_on_two_streams_at_once(pkg, orc, dev):
+@pytest.mark.parametrize("K", [576, 512])
+def test_q8_linear_on_two_streams_at_once(pkg, orc, dev, K):
     """The op-level entry points keep their intermediate buffers (here the
-    quantized activations of an fp32 input) per (device, stream): two streams
-    that issue calls at the same time, with different row counts and no
-    synchronization between them, each get the oracle's result bit for bit."""
-    K, N = 512, 512
-    shapes = {"a": 2048, "b": 96}
-    print("q8_linear on two streams: rows " + ", ".join(map(str, shapes.values())), flush=True)
-    w, mult, bias = None, None, None
-    inputs, refs = {}, {}
-    for i, (key, M) in enumerate(shapes.items()):
-        a, w_i, mult_i, bias_i = pkg.gemm_inputs(M, K, N, seed=100 + i)
-        if w is None:
-            w, mult, bias = w_i, mult_i, bias_i
-        inputs[key] = a
-        refs[key] = orc.linear_forward(a, w, mult, bias, threads=16)[0]
-    dw, dm, db = (dev.DeviceArray.from_host(x) for x in (w, mult, bias))
+    quantized activations of an fp32 input, K = 576) per (device, stream): two
+    streams that issue calls at the same time, with different row counts that
+    grow on the way and no synchronization between them, each get the oracle's
+    result bit for bit.  Rows of K = 512 need no such buffer."""
+    N = 512
+    shapes = {"a": [300, 2048, 2048, 900], "b": [96, 500, 96, 500]}
+    print(f"q8_linear on two streams: K={K} rows {shapes}", flush=True)
+    x, w, mult, bias = pkg.gemm_inputs(2 * 2048, K, N, seed=100)
+    ref = orc.linear_forward(x, w, mult, bias, threads=16)[0]
+    dw, dm, db = (dev.DeviceArray.from_host(v) for v in (w, mult, bias))
+    first = {"a": 0, "b": 2048}  # each stream's own rows
     streams = {k: dev.Stream() for k in shapes}
     try:
-        din = {k: dev.DeviceArray.from_host(inputs[k]) for k in shapes}
-        outs = {k: [dev.DeviceArray.zeros((shapes[k], N), np.float32) for _ in range(4)] for k in shapes}
+        din = {k: [dev.DeviceArray.from_host(x[first[k]:first[k] + m]) for m in shapes[k]] for k in shapes}
+        outs = {k: [dev.DeviceArray.zeros((m, N), np.float32) for m in shapes[k]] for k in shapes}
         err = dev.DeviceArray.zeros(1, np.int32)
+        dev.synchronize()
         for rep in range(4):  # interleaved, never waiting
             for k in shapes:
-                dev.q8_linear(din[k], dw, dm, db, None, outs[k][rep], err=err, stream=streams[k].handle)
+                dev.q8_linear(din[k][rep], dw, dm, db, None, outs[k][rep], err=err, stream=streams[k].handle)
         for st in streams.values():
             st.sync()
         assert err.host()[0] == 0
         for k in shapes:
-            for rep in range(4):
-                assert np.array_equal(outs[k][rep].host().view(np.uint32), refs[k].view(np.uint32)), (k, rep)
+            for rep, m in enumerate(shapes[k]):
+                want = ref[first[k]:first[k] + m]
+                assert np.array_equal(outs[k][rep].host().view(np.uint32), want.view(np.uint32)), (k, rep)
     finally:
         for st in streams.values():
+            st.close()
+
+
+def test_vocab_argmax_on_two_streams_at_once(dev):
+    """The argmax partials are such a buffer too: 512 and 40 rows on two streams."""
+    K, V = 256, 8000
+    rng = np.random.default_rng(51)
+    emb = rng.integers(-127, 128, (V, K)).astype(np.int8)
+    mult, bias = rng.uniform(50, 100, V).astype(np.float32), rng.standard_normal(V).astype(np.float32)
+    D = dev.DeviceArray
+    weights = [D.from_host(v) for v in (emb, mult, bias)]
+    streams = [dev.Stream() for _ in range(2)]
+    try:
+        calls = []
+        for st, M in zip(streams, (512, 40)):
+            xq, xa = rng.integers(-127, 128, (M, K)).astype(np.int8), rng.uniform(1.0, 300.0, M).astype(np.float32)
+            acc = (xq.astype(np.float32) @ emb.astype(np.float32).T)  # below 2^24: exact
+            ref = acc * (np.float32(1) / (xa[:, None] * mult[None, :])) + bias
+            ref[:, [1, *range(7, 39)]] = -np.inf
+            calls.append((st, D.from_host(xq), D.from_host(xa), [D.zeros(M, np.int32) for _ in range(8)], ref.argmax(1)))
+        dev.synchronize()
+        for rep in range(8):
+            for st, xq, xa, toks, _ in calls:
+                dev.vocab_argmax(xq, xa, *weights, toks[rep], stream=st.handle)
+        for st in streams:
+            st.sync()
+        for _, _, _, toks, want in calls:
+            for tok in toks:
+                assert np.array_equal(tok.host(), want)
+    finally:
+        for st in streams:
             st.close()
 
 
@@ -631,7 +661,7 @@ def test_attention_edges(pkg, orc, dev):
 ])
 def test_packed_attention_units(pkg, orc, dev, heads, head_dim, bf16, lens):
     """Packed self-attention against the oracle, bit for bit, with row strides
-    wider than the rows and one sequence holding infinite and NaN keys."""
+    wider than the rows and infinite and NaN elements."""
     print(f"packed attention heads={heads} head_dim={head_dim} bf16={bf16} n={len(lens)}", flush=True)
     rng = np.random.default_rng(41)
     lens = np.array(lens, np.int64)
@@ -640,8 +670,11 @@ def test_packed_attention_units(pkg, orc, dev, heads, head_dim, bf16, lens):
     ld = (d + 15) // 8 * 8
     wide = [rng.standard_normal((T, ld)).astype(np.float32) for _ in range(3)]
     wide[0][:: 3] *= 40.0  # scores far apart: exponentials down to denormals and zero
-    r = int(cu[1])
-    wide[1][r, 0], wide[1][r, head_dim - 1] = np.inf, np.nan
+    # an infinite key element (scores of either sign, by the query's), a NaN one and an
+    # infinite value, each in a head and sequence of its own
+    wide[1][int(cu[1]), 0] = np.inf
+    wide[1][int(cu[3]) - 1, head_dim] = np.nan
+    wide[2][int(cu[3]), 2] = -np.inf
     if bf16:
         dev_in = [dev.DeviceArray.from_host(pkg.synthetic.bf16_round(x)) for x in wide]
         wide = [pkg.synthetic.bf16_to_f32(pkg.synthetic.bf16_round(x)) for x in wide]
