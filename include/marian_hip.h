@@ -457,7 +457,8 @@ int marian_hip_residual_layer_norm(const float* x, const float* r, const float* 
  * n_seqs > 0 declares packed self-attention: the query rows are the key rows
  * (row i lies in [cu_k[s], cu_k[s+1]) for s = seq_of_row[i]), cu_k has
  * n_seqs + 1 entries, rows = cu_k[n_seqs]; then ranges of at most 512 keys
- * run on the kernel that stages each sequence's keys once per 16 or 64 queries.
+ * run on the kernel that stages each sequence's keys once per 16 or 64 queries
+ * (few long rows excepted).
  * n_seqs = 0: one (row, head) wave each, for any query/key pairing. */
 int marian_hip_attention(const void* q, int64_t ldq, const void* k, const void* v, int64_t ldkv,
                          const int32_t* seq_of_row, const uint32_t* cu_k, int64_t n_seqs,

@@ -506,7 +506,8 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s, hipEvent_t ev_star
                  !(a.qmult < __builtin_huge_valf())))
     return hipErrorInvalidValue;
   // Packed self-attention: keys staged once per query tile.
-  if (a.mode == ATT_SEQ && a.n_seqs > 0 && a.max_keys <= kSeqMaxKeys) return launch_attention_seq(a, s);
+  if (a.mode == ATT_SEQ && a.n_seqs > 0 && a.max_keys <= kSeqMaxKeys && attention_seq_wins(a))
+    return launch_attention_seq(a, s);
   // Decode launches cover few rows: one round trip per row matters more
   // than occupancy.  Encoder launches keep the lighter register budget.
   hipEvent_t e0 = ev_start, e1 = ev_stop;

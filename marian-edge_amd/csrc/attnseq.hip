@@ -575,6 +575,16 @@ bool seq_buffer_rows(const AttnArgs& a) {
 
 }  // namespace
 
+// One wave per (row, head) is faster where few long rows leave even the 4-query
+// units' eight chunks unhidden: 424 rows of 257-512 keys with 1 head 18.0 | 26.9 us
+// here, with 2 20.4 | 26.9, with 3 (1284 pairs) 24.5 | 26.8, with 4 (1712) 27.9 | 26.7.
+// The average length tells such calls from short sequences under a max_keys
+// far above them.  That kernel addresses all keys of a range by 32 bits.
+bool attention_seq_wins(const AttnArgs& a) {
+  return a.max_keys <= 256 || (int64_t)a.rows * a.heads > 1536 || a.rows <= 128 * (int64_t)a.n_seqs ||
+         !seq_buffer_rows(a) || a.ldkv >= (int64_t(1) << 32) / (kSeqMaxKeys * 4);
+}
+
 hipError_t launch_attention_seq(const AttnArgs& a, hipStream_t s) {
   if (a.mode != ATT_SEQ || a.n_seqs <= 0 || a.max_keys <= 0 || a.max_keys > kSeqMaxKeys || !a.cu ||
       (int64_t)a.n_seqs * a.heads > 0x7fffffff || (int64_t)a.rows * a.heads > 0x7fffffff)

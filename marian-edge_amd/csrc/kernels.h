@@ -331,6 +331,7 @@ hipError_t launch_attention(const AttnArgs& a, hipStream_t s, hipEvent_t ev_star
 // Packed self-attention (a.n_seqs > 0) over at most kSeqMaxKeys keys, one
 // workgroup per 64 (few rows: 16) queries of a (sequence, head).
 constexpr int kSeqMaxKeys = 512;
+bool attention_seq_wins(const AttnArgs& a);  // against one wave per (row, head)
 hipError_t launch_attention_seq(const AttnArgs& a, hipStream_t s);
 
 // Decode attention block (one launch per attention sublayer on steps with few

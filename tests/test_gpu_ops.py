@@ -655,6 +655,8 @@ def test_attention_edges(pkg, orc, dev):
     (4, 64, False, [257, 320, 321, 511, 512, 3, 30]),
     (4, 64, False, [257, 320, 321, 511, 512, 3, 30] * 3),
     (4, 48, True, [400, 17, 449] * 8),
+    # few long rows: one wave per (row, head), and right past that
+    (1, 64, False, [300, 3, 500, 7]), (2, 48, True, [400, 200, 9, 100]), (2, 64, False, [400, 300, 60, 9]),
     # more sequences than one pass of the lookup, and more than it takes
     (4, 64, False, [1 + (7 * i) % 50 for i in range(600)]),
     (2, 64, False, [1 + (11 * i) % 70 for i in range(1030)]),
