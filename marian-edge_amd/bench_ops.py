@@ -7,10 +7,10 @@ varlen attention workload, timed from a rocprofv3 kernel trace of this script
         python3 marian-edge_amd/bench_ops.py run --out DIR/ops_run.json
     python3 marian-edge_amd/bench_ops.py summarize DIR/ops_run.json DIR/ops_kernel_trace.csv
 
-`run` executes every case `reps` times back to back and records, in call
-order, how many kernels each call dispatches.  `summarize` walks the trace's
-marian-hip dispatches in start order, attributes them to the recorded calls,
-and reports per case the median device time of one call (the sum of its
+`run` executes every case `reps` times back to back and records the cases in
+call order.  `summarize` walks the trace's marian-hip dispatches in start order,
+attributes them to the recorded calls (a call ends with its first kernel that is
+not a row quantization), and reports per case the median device time of one call (the sum of its
 kernels' durations), the algorithmic bytes and the achieved fraction of the
 MI355X's 8 TB/s HBM peak (and of the 5.0 POP/s dense int8 MFMA peak).
 
@@ -22,7 +22,7 @@ Cases:
     per-column scale, i32 + fp32 out); bias reads are 4N more and counted.
   * Varlen attention: 256 packed sentences with lengths ~ lognormal(3.2, 0.6)
     clipped to [4, 256], 8 heads x 64, Q/K/V fp32 and bf16, as packed
-    self-attention (the query-tile list, then the key-staging kernel).
+    self-attention (the key-staging kernel).
     Algorithmic bytes 3 * T * d * b + 4 * T * d (Q, K, V in their type, fp32
     O out).  Also as cross-attention at decode shape: one query per sentence
     (its first row's Q) over the sentence's packed K/V, one wave per (query,
@@ -69,7 +69,7 @@ def run(out_path: str, reps: int) -> None:
                 dev.q8_linear(x, dw, dm, db, oi, of)
             dev.synchronize()
             cases.append(dict(label=f"q8_linear K={K} N={N} M={M}", kind="gemm", M=M, K=K, N=N,
-                              calls=reps, kernels_per_call=2,
+                              calls=reps,
                               bytes=4 * M * K + K * N + 8 * N + 8 * M * N, flops=2 * M * N * K))
             for t in (x, dw, dm, db, oi, of):
                 t.free()
@@ -92,9 +92,8 @@ def run(out_path: str, reps: int) -> None:
             dev.attention(dq, dk, dv, dseq, dcu, do, heads=d // 64, max_keys=lmax, bf16=bf16)
         dev.synchronize()
         # Q, K, V read in their type, O written in fp32.
-        # Two kernels per call: the query-tile list, then the attention.
         cases.append(dict(label=f"attention {'bf16' if bf16 else 'fp32'} T={T}", kind="attention",
-                          T=T, calls=reps, kernels_per_call=2,
+                          T=T, calls=reps,
                           bytes=3 * T * d * b + 4 * T * d, flops=4 * d * int((np.diff(cu.astype(np.int64)) ** 2).sum())))
         for t in (dq, dk, dv, dseq, dcu, do):
             t.free()
@@ -111,7 +110,7 @@ def run(out_path: str, reps: int) -> None:
         dev.synchronize()
         # K and V of every sentence read once, B queries in, B fp32 rows out.
         cases.append(dict(label=f"cross-attention {'bf16' if bf16 else 'fp32'} B={B} T={T}",
-                          kind="attention", T=T, calls=reps, kernels_per_call=1,
+                          kind="attention", T=T, calls=reps,
                           bytes=2 * T * d * b + B * d * b + 4 * B * d, flops=4 * d * T))
         for t in (dq, dk, dv, dseq, dcu, do):
             t.free()
@@ -367,12 +366,18 @@ def summarize(run_path: str, trace_path: str, counter_csv: str | None = None) ->
             if "mh::" in r["Kernel_Name"]:
                 rows.append((int(r["Start_Timestamp"]), int(r["End_Timestamp"]), r["Kernel_Name"]))
     rows.sort()
-    need = sum(c["calls"] * c["kernels_per_call"] for c in spec["cases"])
-    if len(rows) != need:
-        raise SystemExit(f"trace holds {len(rows)} marian-hip dispatches, the run made {need}")
+    calls = []  # each call's dispatches
+    for i, (_, _, name) in enumerate(rows):
+        if not calls or calls[-1][1]:
+            calls.append(([], False))
+        calls[-1][0].append(i)
+        calls[-1] = (calls[-1][0], "k_quantize_rows" not in name)
+    need = sum(c["calls"] for c in spec["cases"])
+    if len(calls) != need:
+        raise SystemExit(f"trace holds {len(calls)} calls, the run made {need}")
     ops = _mfma_ops_per_dispatch(counter_csv) if counter_csv else None
-    if ops is not None and len(ops) != need:
-        raise SystemExit(f"counter file holds {len(ops)} marian-hip dispatches, the run made {need}")
+    if ops is not None and len(ops) != len(rows):
+        raise SystemExit(f"counter file holds {len(ops)} marian-hip dispatches, the trace {len(rows)}")
     head = "| case | kernels | median us / call | algorithmic MB | GB/s | frac of 8 TB/s | int8 MFMA frac |"
     rule = "|---|---|---:|---:|---:|---:|---:|"
     if ops is not None:
@@ -384,10 +389,11 @@ def summarize(run_path: str, trace_path: str, counter_csv: str | None = None) ->
         per_call, per_ops = [], []
         names = set()
         for _ in range(c["calls"]):
-            ks = rows[i:i + c["kernels_per_call"]]
+            at = calls[i][0]
+            ks = [rows[k] for k in at]
             if ops is not None:
-                per_ops.append(sum(ops[i:i + c["kernels_per_call"]]))
-            i += c["kernels_per_call"]
+                per_ops.append(sum(ops[k] for k in at))
+            i += 1
             per_call.append(sum(e - s for s, e, _ in ks) / 1000.0)
             names.update(n.replace("mh::(anonymous namespace)::", "").replace("void ", "").split("(")[0]
                          for _, _, n in ks)
