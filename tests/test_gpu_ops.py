@@ -648,6 +648,8 @@ def test_attention_edges(pkg, orc, dev):
     (8, 64, False, [1, 15, 16, 17, 31, 32, 33, 48, 49, 63, 64, 65, 96, 97, 128, 129, 192, 193, 255, 256, 7] * 3),
     (8, 48, True, [256, 1, 33, 100, 16, 32]),
     (8, 48, True, [256, 1, 33, 100, 16, 32] * 12),
+    # few rows: one long sequence among short ones, odd and even numbers of query tiles
+    (8, 64, False, [256] + [20] * 31), (8, 64, True, [5] * 9 + [239] + [33] * 6), (4, 48, False, [20] * 30 + [512, 1]),
     # heads that leave a shared workgroup's last places empty
     (3, 64, True, [5, 16, 20, 32, 40, 130] * 50),
     (5, 48, False, [16, 17, 64, 65] * 50),
