@@ -38,11 +38,13 @@
 //
 // Measured (before -> now, us): 256 sentences, lengths lognormal(3.2, 0.6), 8
 // heads of 64, fp32 (7405 rows): 59.6 -> 36; 48 segments of 96-256 rows, bf16
-// (8800 rows): 196 -> 96; 54 sentences (1390 rows) 14.9 -> 12.4; one of 15 rows
+// (8800 rows): 196 -> 96; 54 sentences (1390 rows) 14.9 -> 11.9; one of 15 rows
 // 7.6 -> 5.2; 24 sequences of 257-512 rows (9569; one wave per (row, head)
 // before) 851 -> 216.
 #include "device_common.h"
 #include "kernels.h"
+
+#include <algorithm>
 
 namespace mh {
 namespace {
@@ -54,16 +56,18 @@ typedef uint32_t u32u __attribute__((aligned(1)));
 constexpr int kSeqWaves = 4;                   // waves per workgroup
 // (row, head) pairs up to which a wave takes 4 queries instead of 16, by the
 // scores a wave holds (sweep of 8 heads, us with 4 | 16 queries: sentences, 2867
-// rows 20.3 | 22.8, 4393 25.9 | 24.8; segments of 96-256, 2241 rows 32.9 | 40.6,
-// 3528 50.4 | 50.7, 4315 54.6 | 51.9; 257-512 keys, 1697 rows 56.9 | 70.4, 2388
-// 72.5 | 80.3, 3073 84.8 | 78.2).
+// rows 20.1 | 22.6, 4393 24.8 | 24.6; segments of 96-256, 2241 rows 33.5 | 40.6,
+// 3528 54.1 | 50.7, 4315 56.4 | 51.7; 257-512 keys, 1697 rows 58.2 | 70.2, 2388
+// 75.7 | 80.6, 3073 85.8 | 78.1).
 constexpr int64_t kSeqFewRows256 = 32768, kSeqFewRows512 = 20480;
-// Workgroups up to which that holds: max_keys may be far above the lengths, and
-// each 4096 that find nothing cost 1.2 us, where with 16 queries the lengths
-// decide (1024 sequences of 4 rows, max_keys 4: 8192 workgroups, 25.2 us with 4
-// queries | 44.3 with 16; max_keys 64: 32768, 30.9 | 44.8; 256: 131072, 60.4 |
-// 44.7; 300 of 8 rows, 19200: 17.0 | 14.9; 38400: 22.4 | 15.0).
-constexpr int64_t kSeqFewGroups = 24576;
+// Workgroups up to which that holds, and workgroups per sequence past them:
+// max_keys may be far above the lengths, and each 4096 that find nothing cost
+// 1.6 us; with 16 queries the lengths decide, but finding a unit costs more the
+// more sequences there are (us with 4 | 16: 300 of 8 rows, 9600 workgroups 15.2 |
+// 14.9, 19200 19.0 | 14.9, 38400 27.1 | 15.0; 500 of 4 rows, 32000 25.6 | 21.1;
+// 1024 of 4 rows, 8192 25.2 | 44.4, 32768 35.0 | 44.6, 131072 76.2 | 44.7; 128
+// sentences, 16384 27.4 | 28.8).
+constexpr int64_t kSeqFewGroups = 16384, kSeqFewGroupsPer = 48;
 constexpr int kSeqFindMax = 1024;              // sequences up to which a workgroup finds its unit itself
 constexpr int kSeqRow = kHeadDim + 4;          // padded LDS row (floats), 16-byte aligned
 
@@ -342,15 +346,16 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
     h0 = __builtin_amdgcn_readfirstlane(h0);
     tiles = CH;  // the last class's
   } else if constexpr (QW == 4) {
-    // Workgroups go round the XCDs and their 32 CUs in order: a sequence's heads
-    // lie on different XCDs, its query tiles on neighbouring CUs (with the tiles
-    // slowest, 32 sequences put all tiles of a long one on one CU: 32 sentences,
-    // 775 rows, 22.4 us, so 10.5).  With an even number of tiles each sequence
-    // starts one tile on, or the first tiles of short ones would meet likewise.
+    // Workgroups go round the 8 XCDs and their 32 CUs in order: a sequence's heads
+    // lie on different XCDs, and high query tiles, which only long sequences have,
+    // go first.  A sequence's tiles are heads * n_seqs workgroups apart, so the one
+    // 256 / gcd(heads * n_seqs, 256) on would come to the first's CU: each such
+    // group of tiles starts one sequence on (32 sequences, 775 rows, 8 heads:
+    // 22.5 us without, 10.1 with).
     h0 = blockIdx.x;
-    sq = blockIdx.z;
-    tiles = gridDim.y;
-    qt = (blockIdx.y + (tiles & 1 ? 0 : sq)) % tiles;
+    tiles = gridDim.z;
+    qt = tiles - 1 - blockIdx.z;
+    sq = (blockIdx.y + (blockIdx.z >> (8 - __builtin_ctz(a.heads * a.n_seqs | 256)))) % a.n_seqs;
   } else {
     // Every sequence's heads lie on different XCDs; the heads go slowest, or
     // whole XCDs would idle where short sequences' heads exit (below).
@@ -373,8 +378,8 @@ __global__ __launch_bounds__(64 * kSeqWaves, QW == 4 ? 4 : (CH <= 4 ? 3 : 2)) vo
   const int Lc = min(L, 64 * CH);  // a longer range is cut to its first keys (and flagged)
   const int nch = (Lc + 63) >> 6;
   // A unit's time grows with its chunks, and with few rows the longest units
-  // decide the call: they issue first (64 sentences 16.2 -> 15.2 us, 12 segments
-  // 36.7 -> 33.1, 6 segments 20.7 -> 21.3; within 1% where the chip is full).
+  // decide the call: they issue first (112 sentences 21.2 -> 19.9 us, 8 segments
+  // 30.3 -> 28.3; 6 segments and where the chip is full within 1%).
   if (nch >= 4)
     __builtin_amdgcn_s_setprio(3);
   else if (nch == 3)
@@ -598,13 +603,14 @@ hipError_t launch_attention_seq(const AttnArgs& a, hipStream_t s) {
       (int64_t)a.n_seqs * a.heads > 0x7fffffff || (int64_t)a.rows * a.heads > 0x7fffffff)
     return hipErrorInvalidValue;
   const bool gen = !seq_buffer_rows(a);
+  const int64_t groups = (int64_t)a.n_seqs * a.heads * ((a.max_keys + 4 * kSeqWaves - 1) / (4 * kSeqWaves));
   const bool few = !gen && (int64_t)a.rows * a.heads <= (a.max_keys <= 256 ? kSeqFewRows256 : kSeqFewRows512) &&
-                   (int64_t)a.n_seqs * a.heads * ((a.max_keys + 4 * kSeqWaves - 1) / (4 * kSeqWaves)) <= kSeqFewGroups;
+                   groups <= std::max(kSeqFewGroups, kSeqFewGroupsPer * a.n_seqs);
   const int tq = kSeqWaves * (few ? 4 : 16);
   // Units: at most heads / 4 + 7 / 256 heads L of a sequence of L rows (equal at 65 rows).
   const int64_t units = (int64_t)a.n_seqs * ((a.heads + 3) / 4) + ((int64_t)a.rows * a.heads * 7 + 255) / 256;
   const uint32_t tiles = (a.max_keys + tq - 1) / tq;
-  const dim3 grid = few                         ? dim3(a.heads, tiles, a.n_seqs)
+  const dim3 grid = few                         ? dim3(a.heads, a.n_seqs, tiles)
                     : a.n_seqs <= kSeqFindMax ? dim3((uint32_t)units)
                                                 : dim3(a.n_seqs * a.heads, tiles);
   if (gen)

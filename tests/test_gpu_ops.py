@@ -801,6 +801,7 @@ def test_packed_attention_row_strides(pkg, orc, dev, heads, head_dim, bf16, lens
     (4, 64, False, [600, 20] * 16, 400),
     # far above the lengths: launches of many workgroups without a query
     (8, 64, False, [3, 17] * 120, 256), (8, 48, True, [1, 40] * 45, 512), (4, 64, False, [1, 4, 7] * 400, 256),
+    (8, 48, True, [1, 40] * 30, 512), (4, 64, False, [1, 4, 7] * 400, 128),
 ])
 def test_packed_attention_max_keys_off_the_lengths(pkg, orc, dev, heads, head_dim, bf16, lens, max_keys):
     """Sequences longer than max_keys (every row is written, over all its keys up to
