@@ -501,16 +501,23 @@ hipError_t launch_gemm_tile(const GemmArgs& g, const Epilogue& e, hipStream_t s)
   //   past one round of 128x128 tiles their outputs count without the padding:
   //     12000 x 300 (K 2048; 282 tiles, 220 without) 20.0 / 24.4;
   //   from 2048 256x128 tiles (eight a CU) the largest: 4096 x 32000 175 / 157 / 134.
-  // Both outputs store twice as much per product: past two 128x128 tiles a CU the
-  // small ones win while a tile's sums are short (us a call, 64x64 / 128x128, the
-  // kernel before in brackets): 5504 x 1536 (K 512; 516 tiles) 17.3 / 22.5 (20.5),
-  // 12800 x 1536 33.0 / 35.7 (39.1), (K 1024) 5544 22.5 / 26.6 (25.5), 8528 (804
-  // tiles) 32.5 / 32.3 (35.8); 16640 x 512 (K 2048) 40.5 / 40.2 (42.2).
+  // Both outputs make a barely started third round of 128x128 tiles (two a CU)
+  // long, and 64x64 tiles win while their sums are short (us a call, 64x64 /
+  // 128x128, the kernel before in brackets): 5504 x 1536 (K 512; 516 tiles) 17.3 /
+  // 22.5 (20.5), 5600 x 2048 (704) 20.5 / 23.7 (24.1), 8000 x 2048 (K 640; 1008)
+  // 34.1 / 33.8 (36.1), 5544 x 1536 (K 1024; 528) 22.5 / 26.6 (25.5), 11464 x 1000
+  // (720) 32.0 / 28.9 (37.6), 16640 x 512 (K 2048; 520) 40.5 / 40.2 (42.2).
+  // Where they go through the caches (rows that are not whole 64-byte pieces), the
+  // largest tiles win as soon as the last cache cannot hold them, 256 MB or 2048
+  // 128x128 tiles (128x128 / 256x128): 16384 x 2300 (K 512) 92.7 / 70.5 (108), 15072 x
+  // 2500 (K 1024) 120 / 94.3 (114), 37680 x 1000 (K 640) 113 / 91.1 (89.9).
   const auto tiles = [&](int64_t bm, int64_t bn) { return ((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
-  const bool few_sums = g.K <= 640 || (g.K <= 1024 && tiles(128, 128) <= 768);
-  if (e.out && e.out_i32 && few_sums && tiles(128, 128) > 512) return launch_tile<64, 64, 2, 2, 2>(g, e, 1024, s);
-  const bool one_round = tiles(128, 128) >= 224 && tiles(128, 128) <= 256;
   if (tiles(256, 128) >= 2048) return launch_tile<256, 128, 4, 2, 2>(g, e, 256, s);
+  if (e.out && e.out_i32 && tiles(128, 128) > 512 && tiles(128, 128) <= (g.K <= 640 ? 768 : 640) && g.K <= 1024)
+    return launch_tile<64, 64, 2, 2, 2>(g, e, 1024, s);
+  if (e.out && e.out_i32 && !tile_streams(g, e) && tiles(128, 128) >= 2048)
+    return launch_tile<256, 128, 4, 2, 2>(g, e, 256, s);
+  const bool one_round = tiles(128, 128) >= 224 && tiles(128, 128) <= 256;
   if (one_round || (int64_t)g.M * g.N >= 224 * 128 * 128) return launch_tile<128, 128, 2, 4, 2>(g, e, 1 << 30, s);
   return launch_tile<64, 64, 2, 2, 2>(g, e, 1024, s);
 }
